@@ -281,9 +281,6 @@ int check_raster_status(const rvs_k::RasterWS& ws, const rvs_k::BatchDims& d, ui
     uint32_t st[4];
     HIP_TRY(hipMemcpyAsync(st, ws.status, sizeof st, hipMemcpyDeviceToHost, s), "status copy");
     HIP_TRY(hipStreamSynchronize(s), "stream sync");
-    if (st[3])
-        return fail(RVS_E_TIMEOUT, "inpainting: a bounded wait between strip solvers gave up; the launch set's "
-                                   "results are not valid");
     if (st[1]) {
         if (needed_cap) *needed_cap = st[2];
         if (st[2] == 0xffffffffu)
@@ -533,7 +530,7 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
         s = sf;
     }
     rvs_k::InpaintWS iws = rvs_k::inpaint_ws_carve(base + P.inpaint, d.npx, n_views, P.max_w, P.max_h);
-    iws.fail = ws.status + 3;   // a bounded wait of the inpainting that gave up
+    iws.count = ws.status + 5;  // zeroed with the launch set's status
     iws.rflags = ws.tile_enc;   // tiles the raster left without holes or deferred pixels are skipped
     HIP_TRY(rvs_k::launch_inpaint(dviews, n_views, P.max_w, P.max_h, iws, nullptr, s), "inpaint");
     prof_mark(4, s);
@@ -800,6 +797,7 @@ int rvs_inpaint(float* color, const float* quality, int w, int h, void* workspac
     rvs_k::ViewDesc* dv = (rvs_k::ViewDesc*)workspace;
     const rvs_k::InpaintWS ws =
         rvs_k::inpaint_ws_carve((char*)workspace + align256(sizeof(rvs_k::ViewDesc)), (size_t)w * h, 1, w, h);
+    HIP_TRY(rvs_k::launch_reset_u32(ws.count, 1, s), "reset");
     HIP_TRY(rvs_k::launch_upload(&vd, sizeof vd, dv, s), "view upload");
     HIP_TRY(rvs_k::launch_inpaint(dv, 1, w, h, ws, map_out, s), "inpaint");
     return RVS_OK;

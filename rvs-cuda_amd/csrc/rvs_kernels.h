@@ -84,8 +84,8 @@ struct RasterWS {
                              // pixel (blending launches); written by every tile
     float* rbuf;             // [rbuf_tiles][source][tile pixel][5] the replay's per-source colour,
                              // depth and validity of deferred pixels
-    uint32_t* status;        // [0] n_deferred, [1] list overflow, [2] entries (saturated), [3] inpainting
-                             // wait gave up, [4] work items
+    uint32_t* status;        // [0] n_deferred, [1] list overflow, [2] entries (saturated), [4] work items,
+                             // [5] inpainting tiles with holes
 };
 
 struct BatchDims {
