@@ -34,6 +34,14 @@ constexpr int kRasterGroup = 4;     // sources rasterised together in k_raster's
 constexpr int kRasterGroupMulti = 4; // sources per phase of the looping instantiation (more sources)
 constexpr int kRasterCache = 1536;  // binned quads per phase whose coverage-pass results stay in LDS
 constexpr int kRasterCacheOne = 960; // the same for launch sets of up to kRasterGroup sources (one phase)
+// k_raster: a triangle with more pixels of a tile than this in its box is shared by the lanes of a
+// wave.  8 views of 1920x1080 / one 8192x4096 equirectangular view, three scenes each, raster ms: 32 pixels
+// 1.17 1.92 1.07 / 12.4 15.3 13.8; 64: 1.22 1.82 1.10 / 10.9 15.8 12.6; 96: 1.27 1.84 1.11 / 10.8 16.1 12.4;
+// never: 1.80 3.00 1.30 / 10.7 18.1 12.2 (magnified triangles of one size fill whole waves near a
+// pole: side by side is as good there until they exceed a wave).
+constexpr int kWidePx = 64;
+constexpr int kWideQueueOne = 100;  // such triangles put off per phase (in the LDS the one-phase blocks leave free)
+constexpr int kWideQueue = 500;     // the same in the looping instantiation
 constexpr int kMaxSourceSide = 65536;  // bins hold quads as (row << 16) | column; also the
                                        // largest target side (tile coordinates fit 16 bits)
 constexpr int kFallbackBlocks = 1024;
