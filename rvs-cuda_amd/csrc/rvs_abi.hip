@@ -98,6 +98,9 @@ void fill_source(PairGeom& g, const rvs_cam* src, const float* tab) {
     g.sw = src->w; g.sh = src->h;
     g.src_erp = src->proj == 1;
     g.sf0 = src->f[0]; g.sf1 = src->f[1]; g.sp0 = src->p[0]; g.sp1 = src->p[1];
+    const bool q = rvs_math::quot_den(g.sf0) && rvs_math::quot_den(g.sf1);
+    g.rsf0 = q ? 1.f / g.sf0 : 0.f;
+    g.rsf1 = q ? 1.f / g.sf1 : 0.f;
     g.tab = tab;
 }
 

@@ -34,6 +34,7 @@ struct PairGeom {
     int sw, sh;
     int src_erp;                 // 1: ERP source, 0: perspective
     float sf0, sf1, sp0, sp1;    // perspective source intrinsics
+    float rsf0, rsf1;            // 1 / sf0, 1 / sf1 when both are in quot_den's range, else 0
     const float* tab;            // ERP source: cos(phi)[sw], sin(phi)[sw], cos(theta)[sh], sin(theta)[sh]
     // raw depth plane (Y plane of the depth file) and its decode parameters
     const void* depth;
@@ -112,9 +113,10 @@ __device__ inline float3 unproject_src(const PairGeom& g, int i, int j) {
     } else {
         if (d > 0.f) {
             const float uu = (float)j + 0.5f, vv = (float)i + 0.5f;
+            const bool q = g.rsf0 != 0.f && quot_num(d);
             x = d;
-            y = -(d / g.sf0) * (uu - g.sp0);
-            z = -(d / g.sf1) * (vv - g.sp1);
+            y = -(q ? quot(d, g.sf0, g.rsf0) : d / g.sf0) * (uu - g.sp0);
+            z = -(q ? quot(d, g.sf1, g.rsf1) : d / g.sf1) * (vv - g.sp1);
         } else {
             x = y = z = __builtin_nanf("");
         }
@@ -149,8 +151,15 @@ __device__ inline float3 project_tgt(const PairGeom& g, float3 p, bool* und = nu
         v = g.v0 + g.dv_dtheta * theta;
     } else {
         if (X > 0.f) {
-            u = g.df0n * Y / X + g.dp0;
-            v = g.df1n * Z / X + g.dp1;
+            const float nu = g.df0n * Y, nv = g.df1n * Z;
+            if (quot_den(X) && quot_num(nu) && quot_num(nv)) {
+                const float r = recip(X);
+                u = quot(nu, X, r) + g.dp0;
+                v = quot(nv, X, r) + g.dp1;
+            } else {
+                u = nu / X + g.dp0;
+                v = nv / X + g.dp1;
+            }
             vd = X;
         } else {
             u = v = vd = __builtin_nanf("");
@@ -361,6 +370,25 @@ __device__ inline void tri_tight(const Tri& T, int& xa, int& xb, int& ya, int& y
     yb = imin(yb, cvt_i32(__builtin_floorf(fminf(maxy - 0.5f + dl, 1e9f))));
 }
 
+// Box of the pixels in columns [x0, x1], rows [y0, y1] (inside the image) that
+// T, loaded, can cover: tri_near_box, else colorize_triangle's box narrowed by
+// tri_tight.  False when it is empty or colorize_triangle returns before it.
+__device__ inline bool tri_box(Tri& T, int out_w, int out_h, int x0, int x1, int y0, int y1, int& xa, int& xb, int& ya,
+                               int& yb) {
+    if (T.den <= 0.f) return false;   // not a NaN
+    if (!tri_near_box(T.A0, T.A1, T.B0, T.B1, T.C0, T.C1, T.den, x0, x1, y0, y1, xa, xb, ya, yb)) {
+        const float3 a = make_float3(T.A0, T.A1, T.dA), b = make_float3(T.B0, T.B1, T.dB),
+                     c = make_float3(T.C0, T.C1, T.dC);
+        if (!tri_setup_geom(T, a, b, c, out_w, out_h)) return false;
+        xa = imax(T.xmin, x0); xb = imin(T.xmax, x1);
+        ya = imax(T.ymin, y0); yb = imin(T.ymax, y1);
+        if (is_finite(T.A0) && is_finite(T.A1) && is_finite(T.B0) && is_finite(T.B1) && is_finite(T.C0) &&
+            is_finite(T.C1))
+            tri_tight(T, xa, xb, ya, yb);
+    }
+    return xa <= xb && ya <= yb;
+}
+
 // Numerators of the barycentric coordinates l1, l2 at pixel (x, y).
 __device__ inline void tri_num(const Tri& T, int x, int y, float& n1, float& n2) {
     const float offset = 0.5f;
@@ -376,6 +404,36 @@ __device__ inline bool tri_cover(const Tri& T, float n1, float n2, float& l1, fl
     l3 = 1.f - l1 - l2;
     const float eps = 1e-6f;
     return l1 >= -eps && l2 >= -eps && l3 >= -eps;
+}
+
+// The same with r = recip(den), den in quot_den's range.  Where a numerator is
+// outside quot_num's range l1 or l2 may differ from the division, but then it
+// is below 2^-20 either way, or the pixel is not covered either way.
+__device__ inline bool tri_cover_r(const Tri& T, float r, float n1, float n2, float& l1, float& l2, float& l3) {
+    l1 = quot(n1, T.den, r);
+    l2 = quot(n2, T.den, r);
+    l3 = 1.f - l1 - l2;
+    const float eps = 1e-6f;
+    return l1 >= -eps && l2 >= -eps && l3 >= -eps;
+}
+
+// Rejection of pixels that tri_cover cannot accept, r as above: l1 and l2 to
+// 4 * 2^-24 relative, so a value below -2e-6 is below -1e-6 in tri_cover (l3's
+// error is at most 5e-7 where l1 and l2 are not below -2e-6 themselves).
+// NaNs are passed over.
+__device__ inline bool tri_outside_r(float r, float n1, float n2) {
+    const float l1 = n1 * r, l2 = n2 * r;
+    return min3f(l1, l2, 1.f - l1 - l2) < -2e-6f;
+}
+
+// The barycentric coordinates of a covered pixel (x, y), bit for bit.
+__device__ inline void tri_bary(const Tri& T, int x, int y, float& l1, float& l2, float& l3) {
+    float n1, n2;
+    tri_num(T, x, y, n1, n2);
+    if (quot_den(T.den) && quot_num(n1) && quot_num(n2))
+        tri_cover_r(T, recip(T.den), n1, n2, l1, l2, l3);
+    else
+        tri_cover(T, n1, n2, l1, l2, l3);
 }
 
 // Barycentric coordinates at pixel (x, y); returns coverage.

@@ -119,8 +119,88 @@ RVS_HD float ff_rcp(float x) {
 #endif
 }
 
+// (int)floor(x), saturating; NaN gives 0.
+RVS_HD int floor_sat_i32(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+#else
+    const float f = std::floor(x);
+    return is_nan(x) ? 0 : f >= 2147483648.0f ? INT_MAX : f < -2147483648.0f ? INT_MIN : (int)f;
+#endif
+}
+
+// Smallest / largest of three numbers (a NaN is passed over).
+RVS_HD float min3f(float a, float b, float c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return std::fmin(std::fmin(a, b), c);
+#endif
+}
+RVS_HD float max3f(float a, float b, float c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return std::fmax(std::fmax(a, b), c);
+#endif
+}
+
 // float -> uint8/uint16 as MSVC emits it (32-bit cvttss2si then truncation)
 RVS_HD uint32_t quantize_u32(float v, unsigned maxv) { return (uint32_t)cvt_i32(v * (float)maxv); }
+
+// Correctly rounded quotients that share a divisor: quot(n, d, recip(d)) is
+// n / d bit for bit for d in quot_den's range and |n| in quot_num's.  One
+// Newton step on a reciprocal within an ulp, then two residual corrections:
+// the same steps a correctly rounded division takes, without its scaling of
+// extreme operands (not needed in these ranges: no operand, residual or
+// result comes near the subnormals) and with the reciprocal's steps paid once
+// per divisor.  VALU issue slots on gfx950: a division 15, recip 6, quot 5.
+// Outside the ranges (a zero numerator included) quot is only near n / d.
+RVS_HD float recip(float d) {
+    const float y = ff_rcp(d);
+    return ffma(ffma(-d, y, 1.0f), y, y);
+}
+RVS_HD float quot(float n, float d, float r) {
+    float q = n * r;
+    q = ffma(ffma(-d, q, n), r, q);
+    return ffma(ffma(-d, q, n), r, q);
+}
+RVS_HD bool quot_den(float d) { return d >= 9.313225746e-10f && d <= 1.099511628e12f; }   // [2^-30, 2^40]
+RVS_HD bool quot_num(float n) {   // [2^-50, 2^60]
+    const float a = fabs_(n);
+    return a >= 8.881784197e-16f && a <= 1.152921505e18f;
+}
+
+// Box [xa, xb] x [ya, yb] of the pixels in columns [x0, x1], rows [y0, y1]
+// that a triangle of positive denominator `den` can cover (empty when it can
+// cover none): pixel centres within 0.07 + 4e-6 s of its extent, s = largest
+// extent + 2 (the argument is with tri_tight).  Returns false, with nothing
+// set, for what that bound does not hold for: thin triangles (den below
+// 2^-14 s^3), huge or non-finite ones.  x0, y0 >= 0.
+// The coordinates are finite here (a non-finite one makes den NaN, or infinite
+// with an infinite s), so hardware minima and a saturating conversion stand in
+// for the reference's ordered minima and cvttss2si (a box left of or above the
+// int range is empty either way).  About 30 VALU instructions against 141
+// of the reference's box and the narrowing after it.
+RVS_HD bool tri_near_box(float A0, float A1, float B0, float B1, float C0, float C1, float den, int x0, int x1, int y0,
+                         int y1, int& xa, int& xb, int& ya, int& yb) {
+    const float minx = min3f(A0, B0, C0), maxx = max3f(A0, B0, C0);
+    const float miny = min3f(A1, B1, C1), maxy = max3f(A1, B1, C1);
+    const float s = max3f(maxx - minx, maxy - miny, 0.f) + 2.f;
+    if (!(den >= 6.103515625e-05f * s * s * s && s <= 65536.f && maxx <= 1e9f && maxy <= 1e9f)) return false;   // 2^-14
+    const float dl = ffma(4e-6f, s, 0.57f), dh = dl - 1.f;
+    xa = imax(x0, -floor_sat_i32(dl - minx));
+    xb = imin(x1, floor_sat_i32(maxx + dh));
+    ya = imax(y0, -floor_sat_i32(dl - miny));
+    yb = imin(y1, floor_sat_i32(maxy + dh));
+    return true;
+}
 
 // ---------------------------------------------------------------------------
 // Exact emulation of  (float) sqrt( ((0.0 + (double)a*a) + (double)b*b) + (double)c*c )

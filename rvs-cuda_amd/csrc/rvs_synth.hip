@@ -101,6 +101,20 @@ __device__ inline uint32_t tile_of_block(uint32_t b, uint32_t ntiles) {
 
 // ------------------------------------------------------------------ quads
 
+// vertex() of the N corners (i + di, j + dj), bit k of ROWS / COLS being di /
+// dj of corner k, one after the other (not unrolled: the evaluation is large
+// and, where a kept window is the rule, rare).
+template <int N, class G>
+__device__ inline void eval_corners(const G& g, int i, int j, uint32_t rows, uint32_t cols, float3 (&v)[N], bool* und) {
+#pragma unroll 1
+    for (int k = 0; k < N; ++k) {
+        const float3 x = vertex(g, i + (int)((rows >> k) & 1u), j + (int)((cols >> k) & 1u), und);
+#pragma unroll
+        for (int m = 0; m < N; ++m)
+            if (m == k) v[m] = x;
+    }
+}
+
 // The (up to four) triangles of source quad (i, j), with the reference's
 // vertex gating (transform.cpp:161-176).  alive bit k set = colorize_triangle
 // is called for slot k and gets past its early returns.
@@ -146,38 +160,31 @@ __device__ inline void quad_build(Quad& Q, const G& g, int i, int j, VF vtx, int
 // quad_build + quad_tiles compute), one triangle at a time; with tv, also the
 // validities of T1 and T2 (0 when not alive or left undecided by the fast
 // path).  False when no triangle can cover a pixel.
-template <class G, class VF>
-__device__ inline bool quad_range_tv(const G& g, int i, int j, VF vtx, int out_w, int out_h, int shift, int& tx0,
-                                     int& tx1, int& ty0, int& ty1, float2* tv) {
+template <class G>
+__device__ inline bool quad_range_tv(const G& g, int i, int j, float3 v00, float3 v01, float3 v10, float3 v11, int out_w,
+                                     int out_h, int shift, int& tx0, int& tx1, int& ty0, int& ty1, float2* tv) {
     if (tv) *tv = make_float2(0.f, 0.f);
-    const float3 v01 = vtx(i, j + 1), v10 = vtx(i + 1, j);
     if (!(v01.z > 0.f && v10.z > 0.f && v01.x > 0.f && v10.x > 0.f)) return false;
     int xmin = INT_MAX, xmax = INT_MIN, ymin = INT_MAX, ymax = INT_MIN;
     auto one = [&](float3 a, float3 b, float3 c, float* tvo) {
         Tri T;
-        if (!tri_setup_geom(T, a, b, c, out_w, out_h)) return;
-        // tiles only where the triangle can cover a pixel (tri_tight; a triangle
-        // that can cover none is never rasterised, so its validity is unused)
-        int xa = T.xmin, xb = T.xmax, ya = T.ymin, yb = T.ymax;
-        tri_tight(T, xa, xb, ya, yb);
-        if (xa <= xb && ya <= yb) {
-            xmin = min(xmin, xa); xmax = max(xmax, xb);
-            ymin = min(ymin, ya); ymax = max(ymax, yb);
-        }
+        tri_load(T, a, b, c);
+        int xa, xb, ya, yb;
+        // a triangle that can cover no pixel is never rasterised
+        if (!tri_box(T, out_w, out_h, 0, out_w - 1, 0, out_h - 1, xa, xb, ya, yb)) return;
+        xmin = min(xmin, xa); xmax = max(xmax, xb);
+        ymin = min(ymin, ya); ymax = max(ymax, yb);
         // fast path only: an undecided validity stays 0 (unknown), and the
         // raster then defers the pixels that depend on it
         if (tvo && !tri_validity_fast(T, g.rescale, *tvo)) *tvo = 0.f;
     };
-    const float3 v00 = vtx(i, j);
     if (v00.z > 0.f && v00.x > 0.f) one(v00, v01, v10, tv ? &tv->x : nullptr);
-    {
-        const float3 v11 = vtx(i + 1, j + 1);
-        if (v11.z > 0.f && v11.x > 0.f) one(v11, v10, v01, tv ? &tv->y : nullptr);
-    }
+    if (v11.z > 0.f && v11.x > 0.f) one(v11, v10, v01, tv ? &tv->y : nullptr);
     if (g.wrap && j == 0) {
-        const float3 l0 = vtx(i, g.sw - 1), l1 = vtx(i + 1, g.sw - 1);
-        one(l0, v00, l1, nullptr);
-        one(v10, l1, v00, nullptr);
+        float3 l[2];   // (i, sw - 1), (i + 1, sw - 1)
+        eval_corners<2>(g, i, g.sw - 1, 2u, 0u, l, nullptr);
+#pragma unroll 1
+        for (int k = 0; k < 2; ++k) one(k ? v10 : l[0], k ? l[1] : v00, k ? v00 : l[1], nullptr);
     }
     if (xmin > xmax) return false;
     tx0 = xmin >> shift; tx1 = xmax >> shift; ty0 = ymin >> shift; ty1 = ymax >> shift;   // boxes start at >= 0
@@ -391,17 +398,24 @@ __device__ inline void unpack_range(uint32_t r, int& tx0, int& tx1, int& ty0, in
 
 // Vertex (row lr, column lc) of a kept work item's vertex block (the counting
 // pass evaluated it with vertex(); the bits are the same).
+__device__ inline float3 load3(const float* p) { return make_float3(p[0], p[1], p[2]); }
 __device__ inline float3 kept_vertex(const float* vb, int lr, int lc) {
-    const float* p = vb + 3 * (lr * (kBinQX + 1) + lc);
-    return make_float3(p[0], p[1], p[2]);
+    return load3(vb + 3 * (lr * (kBinQX + 1) + lc));
 }
 
-// Work index of the kept work item holding quad (i, j) of pair vs, or ~0.
-// (always ~0 when kept items store no vertex windows)
+// Work index of the kept work item holding quad (i, j) of pair vs, or ~0
+// (always ~0 when kept items store no vertex windows).  KEPT: every surviving
+// item is kept.
+template <bool KEPT = false>
 __device__ inline uint32_t kept_index(const RasterWS& ws, const BatchDims& d, uint32_t vs, int i, int j) {
-    if (!d.kept_geom) return 0xffffffffu;
+    if (!KEPT && !d.kept_geom) return 0xffffffffu;
     const uint32_t item = (uint32_t)(i / kBinQY) * d.bins_x + (uint32_t)(j / kBinQX);
     return ws.imap[(size_t)vs * (d.bins_x * d.bins_y) + item];
+}
+
+// Upper left vertex of quad (i, j) in the window of kept item wi.
+__device__ inline const float* kept_quad(const RasterWS& ws, uint32_t wi, int i, int j) {
+    return ws.vbuf + (size_t)wi * (3 * kBinVerts) + 3 * ((i % kBinQY) * (kBinQX + 1) + j % kBinQX);
 }
 
 // Vertex block of quad (i, j) of pair vs when its work item was kept, else null.
@@ -414,6 +428,14 @@ __device__ inline const float* kept_block(const RasterWS& ws, const BatchDims& d
 // pass evaluated them exactly; only alive triangles' values are meaningful).
 __device__ inline float2 kept_validity(const RasterWS& ws, uint32_t wi, int i, int j) {
     return ws.tvq[(size_t)wi * 256 + (uint32_t)((i % kBinQY) * kBinQX + (j % kBinQX))];
+}
+
+// Vertices (i, sw - 1) and (i + 1, sw - 1) of pair vs, every item being kept:
+// from the window of the last quad of the row.
+__device__ inline void kept_seam(const RasterWS& ws, const BatchDims& d, uint32_t vs, int i, int sw, float3 (&l)[2]) {
+    const float* p = kept_quad(ws, kept_index<true>(ws, d, vs, i, sw - 2), i, sw - 2) + 3;
+    l[0] = load3(p);
+    l[1] = load3(p + 3 * (kBinQX + 1));
 }
 
 constexpr uint32_t kTableEmpty = 0xffffffffu;
@@ -448,14 +470,13 @@ __device__ inline int find_slot(const uint32_t* keys, uint32_t t) {
 
 // Tile range [tx0, tx1] x [ty0, ty1] touched by the narrowed bounding boxes
 // of a quad's surviving triangles; false when none can cover a pixel.
-__device__ inline bool quad_tiles(const Quad& Q, int shift, int& tx0, int& tx1, int& ty0, int& ty1) {
+__device__ inline bool quad_tiles(Quad& Q, int out_w, int out_h, int shift, int& tx0, int& tx1, int& ty0, int& ty1) {
     if (!Q.alive) return false;
     int xmin = INT_MAX, xmax = INT_MIN, ymin = INT_MAX, ymax = INT_MIN;
     for (int k = 0; k < 4; ++k)
         if (Q.alive & (1u << k)) {
-            int xa = Q.t[k].xmin, xb = Q.t[k].xmax, ya = Q.t[k].ymin, yb = Q.t[k].ymax;
-            tri_tight(Q.t[k], xa, xb, ya, yb);   // as quad_range_tv: the pixels it can cover
-            if (xa > xb || ya > yb) continue;
+            int xa, xb, ya, yb;   // as quad_range_tv: the pixels it can cover
+            if (!tri_box(Q.t[k], out_w, out_h, 0, out_w - 1, 0, out_h - 1, xa, xb, ya, yb)) continue;
             xmin = min(xmin, xa); xmax = max(xmax, xb);
             ymin = min(ymin, ya); ymax = max(ymax, yb);
         }
@@ -552,19 +573,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
         }
         bool more = false;
         int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;
-        // a kept item also records its quads' triangle validities for the raster
-        // (exact; this pass waits on memory far more than it computes)
-        auto quad_range = [&](auto vtx) {
-            if (stored_geom) {
-                float2 tv;
-                more = quad_range_tv(g, i, j, vtx, vd.w, vd.h, d.tile_shift, tx0, tx1, ty0, ty1, &tv);
-                ws.tvq[(size_t)wi * 256 + tid] = tv;
-            } else {
-                more = quad_range_tv(g, i, j, vtx, vd.w, vd.h, d.tile_shift, tx0, tx1, ty0, ty1, nullptr);
-            }
-        };
+        // a kept item also records its vertices and its quads' triangle validities for the raster
         {
             float* vb = stored_geom ? ws.vbuf + (size_t)wi * (3 * kBinVerts) : nullptr;
+#pragma unroll 1
             for (int k = tid; k < kBinVerts; k += 256) {
                 const int rr = k / (kBinQX + 1), c = k % (kBinQX + 1);
                 const int ii = i0 + rr, jj = j0 + c;
@@ -575,12 +587,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
                 }
             }
             __syncthreads();   // vertices loaded, table cleared
-            if (i < g.sh - 1 && j < g.sw - 1)
-                quad_range([&](int ii, int jj) -> float3 {
-                    const int rr = ii - i0, c = jj - j0;
-                    if (rr >= 0 && rr <= kBinQY && c >= 0 && c <= kBinQX) return V[rr][c];
-                    return vertex(g, ii, jj);
-                });
+            float2 tv = make_float2(0.f, 0.f);
+            if (i < g.sh - 1 && j < g.sw - 1) {
+                const int r = tid / kBinQX, c = tid % kBinQX;
+                more = quad_range_tv(g, i, j, V[r][c], V[r][c + 1], V[r + 1][c], V[r + 1][c + 1], vd.w, vd.h,
+                                     d.tile_shift, tx0, tx1, ty0, ty1, stored_geom ? &tv : nullptr);
+                if (stored_geom) ws.tvq[(size_t)wi * 256 + tid] = tv;
+            }
         }
         auto tile_of = [&](int tx, int ty) { return vd.tile_base + (uint32_t)(ty * vd.tiles_x + tx); };
         auto bin_of = [&](uint32_t t) { return (size_t)t * d.nsrc + s; };
@@ -680,7 +693,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
                            return vertex(g, ii, jj);
                        },
                        vd.w, vd.h, false);
-            more = quad_tiles(Q, d.tile_shift, tx0, tx1, ty0, ty1);
+            more = quad_tiles(Q, vd.w, vd.h, d.tile_shift, tx0, tx1, ty0, ty1);
         } else if (r != kRangeNone) {
             unpack_range(r, tx0, tx1, ty0, ty1);
             more = true;
@@ -863,10 +876,16 @@ __device__ __forceinline__ bool resolve(const G& g, int i, int j, int slot, int 
 #pragma unroll
     for (int k = 0; k < 3; ++k) slot_vertex(slot, k, i, j, g.sw, r[k], cc[k]);
     color3(g, r, cc, col);   // issued first: its loads overlap the vertices'
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+        int rk, ck;
+        slot_vertex(slot, k, i, j, g.sw, rk, ck);
+        const float3 x = (vb && slot < 2) ? kept_vertex(vb, i % kBinQY + (rk - i), j % kBinQX + (ck - j))
+                                          : vertex(g, rk, ck, FAST ? &und : nullptr);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        v[k] = (vb && slot < 2) ? kept_vertex(vb, i % kBinQY + (r[k] - i), j % kBinQX + (cc[k] - j))
-                               : vertex(g, r[k], cc[k], FAST ? &und : nullptr);
+        for (int m = 0; m < 3; ++m)
+            if (m == k) v[m] = x;
+    }
     Tri T;
     if (FAST) {
         tri_setup_geom(T, v[0], v[1], v[2], out_w, out_h);
@@ -875,7 +894,7 @@ __device__ __forceinline__ bool resolve(const G& g, int i, int j, int slot, int 
         tri_setup(T, v[0], v[1], v[2], out_w, out_h, g.rescale);
     }
     float l1, l2, l3;
-    tri_pixel(T, x, y, l1, l2, l3);
+    tri_bary(T, x, y, l1, l2, l3);
     dep = tri_depth(T, l1, l2, l3);
     shape = T.tv;
     c = tri_color(col[0], col[1], col[2], l1, l2, l3);
@@ -896,7 +915,7 @@ __device__ __forceinline__ void resolve_cached(const G& g, int i, int j, int slo
     tri_load(T, a, b, cv);
     T.tv = tv;
     float l1, l2, l3;
-    tri_pixel(T, x, y, l1, l2, l3);
+    tri_bary(T, x, y, l1, l2, l3);
     dep = tri_depth(T, l1, l2, l3);
     shape = tv;
     c = tri_color(col[0], col[1], col[2], l1, l2, l3);
@@ -907,13 +926,14 @@ __device__ __forceinline__ void resolve_cached(const G& g, int i, int j, int slo
 constexpr uint32_t kDeferKey = 0xffffffffu;
 
 // Pushes candidate `id` of triangle T for pixel (x, y) of the tile at (tx0,
-// ty0): the exact coverage test, then the key updates.
+// ty0): the exact coverage test, then the key updates.  r: recip(T.den), or 0
+// when T.den is outside quot_den's range.
 template <int TILE>
-__device__ __forceinline__ void raster_push(const Tri& T, bool special, uint32_t id, int x, int y, int tx0, int ty0,
-                                            unsigned long long* key1, uint32_t* key2) {
+__device__ __forceinline__ void raster_push(const Tri& T, float r, bool special, uint32_t id, int x, int y, int tx0,
+                                            int ty0, unsigned long long* key1, uint32_t* key2) {
     float n1, n2, l1, l2, l3;
     tri_num(T, x, y, n1, n2);
-    if (!tri_cover(T, n1, n2, l1, l2, l3)) return;
+    if (!(r != 0.f ? tri_cover_r(T, r, n1, n2, l1, l2, l3) : tri_cover(T, n1, n2, l1, l2, l3))) return;
     const int p = (y - ty0) * TILE + (x - tx0);
     const float dd = tri_depth(T, l1, l2, l3);
     if (special || !depth_regular(dd)) {
@@ -939,12 +959,26 @@ struct WideQueue {
 
 // Pixels of the tile that triangle T may cover; false when there are none.
 template <int TILE>
-__device__ __forceinline__ bool tile_box(const Tri& T, bool special, int tx0, int ty0, int& xa, int& xb, int& ya,
+__device__ __forceinline__ bool tile_box(Tri& T, int tx0, int ty0, int out_w, int out_h, int& xa, int& xb, int& ya,
                                          int& yb) {
-    xa = max(T.xmin, tx0); xb = min(T.xmax, tx0 + TILE - 1);
-    ya = max(T.ymin, ty0); yb = min(T.ymax, ty0 + TILE - 1);
-    if (!special) tri_tight(T, xa, xb, ya, yb);
-    return xa <= xb && ya <= yb;
+    return tri_box(T, out_w, out_h, tx0, min(out_w, tx0 + TILE) - 1, ty0, min(out_h, ty0 + TILE) - 1, xa, xb, ya, yb);
+}
+
+// Whether pixel (x, y) may pass T's coverage test (r as in raster_push).
+__device__ __forceinline__ bool may_cover(const Tri& T, float r, int x, int y) {
+    float n1, n2;
+    tri_num(T, x, y, n1, n2);
+    return r != 0.f ? !tri_outside_r(r, n1, n2) : !tri_surely_outside(T, n1, n2);
+}
+
+// T's validity: the one the counting pass kept (> 0; KNOWN: it was evaluated
+// there whenever T has a pixel), else the fast path.  False when the fast path
+// leaves it undecided: the pixels the triangle covers are then deferred (T.tv
+// is at least 0 then too).
+template <bool KNOWN>
+__device__ __forceinline__ bool take_validity(Tri& T, float rescale, float tv_known) {
+    T.tv = tv_known;
+    return tv_known > 0.f || (!KNOWN && tri_validity_fast(T, rescale, T.tv));
 }
 
 // Pass over one triangle of a binned quad for the tile at (tx0, ty0): per
@@ -957,17 +991,17 @@ __device__ __forceinline__ bool tile_box(const Tri& T, bool special, int tx0, in
 // it changes nothing).  A finite triangle with more than kWidePx pixels of the
 // tile in its box is left to raster_wide while the queue Q (null: none) has
 // room.
-template <int TILE, class Queue>
+template <int TILE, bool KNOWN, class Queue>
 __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_t id, bool prol_false_possible, int tx0,
                                    int ty0, int out_w, int out_h, float rescale, unsigned long long* key1,
                                    uint32_t* key2, bool undecided, float tv_known, Queue* Q) {
     Tri T;
-    if (!tri_setup_geom(T, a, b, c, out_w, out_h)) return;
-    const bool prol = (a.z > 0.f) || (b.z > 0.f) || (c.z > 0.f);
-    bool special = !finite3(a) || !finite3(b) || !finite3(c) || !is_finite(T.den) ||
-                   (prol_false_possible && !prol) || undecided;
+    tri_load(T, a, b, c);
     int xa, xb, ya, yb;
-    if (!tile_box<TILE>(T, special, tx0, ty0, xa, xb, ya, yb)) return;   // no pixel of this tile can be covered
+    if (!tile_box<TILE>(T, tx0, ty0, out_w, out_h, xa, xb, ya, yb)) return;   // no pixel of this tile can be covered
+    const bool prol = (a.z > 0.f) || (b.z > 0.f) || (c.z > 0.f);
+    // a finite den has finite image coordinates
+    bool special = !is_finite(a.z + b.z + c.z) || !is_finite(T.den) || (prol_false_possible && !prol) || undecided;
     if (Q && !special && (xb - xa + 1) * (yb - ya + 1) > kWidePx) {
         const uint32_t q = atomicAdd(&Q->n, 1u);
         if (q < Queue::cap) {
@@ -975,38 +1009,40 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
             return;
         }
     }
-    if (xb - xa < 8 && yb - ya < 8) {
-        // Two steps, so that lanes with few candidates do not wait through the
-        // exact test of lanes with large boxes: the division-free rejection
-        // marks the candidate pixels of the box (8 x 8 bit mask), then only
-        // those take the exact coverage test and the key updates.
-        uint64_t mask = 0ull;
-        for (int y = ya; y <= yb; ++y)
-            for (int x = xa; x <= xb; ++x) {
-                float n1, n2;
-                tri_num(T, x, y, n1, n2);
-                if (!tri_surely_outside(T, n1, n2)) mask |= 1ull << ((y - ya) * 8 + (x - xa));
+    const float r = quot_den(T.den) ? recip(T.den) : 0.f;
+    const float ex1 = T.B1 - T.C1, ey1 = T.C0 - T.B0, ex2 = T.C1 - T.A1, ey2 = T.A0 - T.C0;   // tri_num's
+    T.tv = -1.f;   // not taken yet
+    // 8 x 8 pixels at a time (nearly every box is smaller), in two steps, so
+    // that lanes with few candidates do not wait through the exact test of
+    // lanes with large boxes: the rejection by approximate barycentrics marks
+    // the candidates (a bit each), then only those take the exact coverage test
+    // and the key updates.
+    for (int y0 = ya; y0 <= yb; y0 += 8)
+        for (int x0 = xa; x0 <= xb; x0 += 8) {
+            const int nx = min(xb - x0, 7), ny = min(yb - y0, 7);
+            const float fx0 = (float)x0 + 0.5f;
+            float fy = (float)y0 + 0.5f;
+            uint64_t mask = 0ull;
+            for (int row = 0; row <= ny; ++row) {
+                const float dy = fy - T.C1, m1 = ey1 * dy, m2 = ey2 * dy;
+                float fx = fx0;
+                uint32_t bits = 0u;
+                for (uint32_t bit = 1u; bit <= 1u << nx; bit <<= 1) {
+                    const float dx = fx - T.C0;
+                    if (!tri_outside_r(r, ex1 * dx + m1, ex2 * dx + m2)) bits |= bit;
+                    fx += 1.f;
+                }
+                mask |= (uint64_t)bits << (row * 8);
+                fy += 1.f;
             }
-        if (!mask) return;   // no candidate pixel: the validity is never needed
-        // a validity kept by the counting pass (> 0), else the fast path; one it
-        // leaves undecided defers the pixels the triangle covers
-        if (tv_known > 0.f) T.tv = tv_known;
-        else if (!tri_validity_fast(T, rescale, T.tv)) special = true;
-        while (mask) {
-            const int bit = __builtin_ctzll(mask);
-            mask &= mask - 1ull;
-            raster_push<TILE>(T, special, id, xa + (bit & 7), ya + (bit >> 3), tx0, ty0, key1, key2);
+            if (!mask) continue;
+            if (T.tv < 0.f && !take_validity<KNOWN>(T, rescale, tv_known)) special = true;
+            while (mask) {
+                const int bit = __builtin_ctzll(mask);
+                mask &= mask - 1ull;
+                raster_push<TILE>(T, r, special, id, x0 + (bit & 7), y0 + (bit >> 3), tx0, ty0, key1, key2);
+            }
         }
-    } else {
-        if (tv_known > 0.f) T.tv = tv_known;
-        else if (!tri_validity_fast(T, rescale, T.tv)) special = true;
-        for (int y = ya; y <= yb; ++y)
-            for (int x = xa; x <= xb; ++x) {
-                float n1, n2;
-                tri_num(T, x, y, n1, n2);
-                if (!tri_surely_outside(T, n1, n2)) raster_push<TILE>(T, special, id, x, y, tx0, ty0, key1, key2);
-            }
-    }
 }
 
 __device__ __forceinline__ float lane_f(float v, int lane) {
@@ -1021,7 +1057,7 @@ __device__ __forceinline__ float lane_f(float v, int lane) {
 // bins: stretched across a depth edge, magnified, or near a pole.
 // Measured: two 3840x2160 views of 11 perspective sources, raster 4.03 -> 3.40
 // ms; 8 views of 1920x1080 of four panoramas 1.80 -> 1.22 ms.
-template <int TILE, int NT, class G, class Queue>
+template <int TILE, int NT, bool KEPT, class G, class Queue>
 __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, const uint32_t* pref, int gs,
                                             uint32_t nwide, const Queue& Q, int wave, int tx0, int ty0, int out_w,
                                             int out_h, unsigned long long (*key1)[NT], uint32_t (*key2)[NT],
@@ -1030,6 +1066,7 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
     for (uint32_t q0 = (uint32_t)wave; q0 < nwide; q0 += 64u * NW) {
         const uint32_t q = q0 + NW * (uint32_t)lane_now();
         Tri T;
+        float tr = 0.f;
         int k = 0, xa = 0, xb = -1, ya = 0, yb = -1, sp = 0;
         uint32_t id = 0u;
         if (q < nwide) {
@@ -1039,21 +1076,27 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
             int i, j;
             unpack_ij(ws.lists[(size_t)boff[k] + (e - pref[k])], i, j);
             const G& g = gv[k];
-            const uint32_t wi = kept_index(ws, d, vs0 + (uint32_t)k, i, j);
-            const float* vb = wi == 0xffffffffu ? nullptr : ws.vbuf + (size_t)wi * (3 * kBinVerts);
-            const float2 tvk = vb ? kept_validity(ws, wi, i, j) : make_float2(0.f, 0.f);
+            const uint32_t wi = kept_index<KEPT>(ws, d, vs0 + (uint32_t)k, i, j);
             // the corners of slot 0 (v00 v01 v10) or 1 (v11 v10 v01); one evaluated
             // here was decided by the fast path when the triangle was queued
             const int slot = (int)(id & 3u);
             bool und = false;
-            auto vtx = [&](int di, int dj) -> float3 {
-                return vb ? kept_vertex(vb, i % kBinQY + di, j % kBinQX + dj) : vertex(g, i + di, j + dj, &und);
-            };
-            const float3 a = vtx(slot, slot), b = vtx(slot, 1 - slot), c = vtx(1 - slot, slot);
-            tri_setup_geom(T, a, b, c, out_w, out_h);
-            tile_box<TILE>(T, false, tx0, ty0, xa, xb, ya, yb);
-            T.tv = slot ? tvk.y : tvk.x;
-            if (!(T.tv > 0.f) && !tri_validity_fast(T, g.rescale, T.tv)) sp = 0x100;
+            float2 tvk = make_float2(0.f, 0.f);
+            float3 c3[3];
+            if (KEPT || wi != 0xffffffffu) {
+                const float* p = kept_quad(ws, wi, i, j);
+                c3[0] = load3(p + (slot ? 3 * (kBinQX + 2) : 0));
+                c3[1] = load3(p + (slot ? 3 * (kBinQX + 1) : 3));
+                c3[2] = load3(p + (slot ? 3 : 3 * (kBinQX + 1)));
+                tvk = kept_validity(ws, wi, i, j);
+            } else {
+                eval_corners<3>(g, i, j, slot ? 3u : 4u, slot ? 5u : 2u, c3, &und);
+            }
+            const float3 a = c3[0], b = c3[1], c = c3[2];
+            tri_load(T, a, b, c);
+            tile_box<TILE>(T, tx0, ty0, out_w, out_h, xa, xb, ya, yb);
+            if (!take_validity<KEPT>(T, g.rescale, slot ? tvk.y : tvk.x)) sp = 0x100;
+            if (quot_den(T.den)) tr = recip(T.den);
         }
         const int m = min(64, (int)((nwide - q0 + NW - 1u) / NW));
         for (int l = 0; l < m; ++l) {
@@ -1068,15 +1111,13 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
             const int n = bw * (__builtin_amdgcn_readlane(yb, l) - wy + 1);
             const int sk = __builtin_amdgcn_readlane(k | sp, l);
             const uint32_t wid = (uint32_t)__builtin_amdgcn_readlane((int)id, l);
-            const float inv = __builtin_amdgcn_rcpf((float)bw);
+            const float inv = __builtin_amdgcn_rcpf((float)bw), r = lane_f(tr, l);
             for (int i = lane_now(); i < n; i += 64) {
                 // row i / bw: i + 1/2 is at least 1 / (2 bw) of a row away from the next one
-                const int r = (int)(((float)i + 0.5f) * inv);
-                const int x = wx + (i - r * bw), y = wy + r;
-                float n1, n2;
-                tri_num(W, x, y, n1, n2);
-                if (!tri_surely_outside(W, n1, n2))
-                    raster_push<TILE>(W, sk >= 0x100, wid, x, y, tx0, ty0, key1[sk & 0xff], key2[sk & 0xff]);
+                const int row = (int)(((float)i + 0.5f) * inv);
+                const int x = wx + (i - row * bw), y = wy + row;
+                if (may_cover(W, r, x, y))
+                    raster_push<TILE>(W, r, sk >= 0x100, wid, x, y, tx0, ty0, key1[sk & 0xff], key2[sk & 0xff]);
             }
         }
     }
@@ -1097,46 +1138,47 @@ struct RasterCache {
 // concatenated bins.  A non-deferred pixel's winner beats every other
 // candidate by more than the float test's error, so any unique id works; equal
 // scores are deferred to the in-order replay.
-template <int TILE, class G, class Cache, class Queue>
-__device__ __forceinline__ void raster_quad(const G& g, uint32_t ij, uint32_t e, int tx0, int ty0, int out_w, int out_h,
-                                   unsigned long long* key1, uint32_t* key2, Cache* C, Queue* Q,
-                                   const RasterWS& ws, const BatchDims& d, uint32_t vs) {
+// gt: any descriptor of the view (target-side fields: the same for all its
+// sources, so they are read once per wave).
+template <int TILE, bool KEPT, class G, class Cache, class Queue>
+__device__ __forceinline__ void raster_quad(const G& g, const G& gt, uint32_t ij, uint32_t e, int tx0, int ty0,
+                                            int out_w, int out_h, unsigned long long* key1, uint32_t* key2, Cache* C,
+                                            Queue* Q, const RasterWS& ws, const BatchDims& d, uint32_t vs) {
     int i, j;
     unpack_ij(ij, i, j);
-    const uint32_t wi = kept_index(ws, d, vs, i, j);
-    const float* vb = wi == 0xffffffffu ? nullptr : ws.vbuf + (size_t)wi * (3 * kBinVerts);
-    const float2 tvk = vb ? kept_validity(ws, wi, i, j) : make_float2(0.f, 0.f);
-    const int li = i % kBinQY, lj = j % kBinQX;
+    const uint32_t wi = kept_index<KEPT>(ws, d, vs, i, j);
     // vertices evaluated here take the fast radius path; an undecided one
     // defers the pixels of the quad's triangles (kept vertices are exact)
     bool und = false;
-    auto vtx = [&](int di, int dj) -> float3 {
-        return vb ? kept_vertex(vb, li + di, lj + dj) : vertex(g, i + di, j + dj, &und);
-    };
-    // vertices are fetched just before their triangles need them; keys
-    // commute, so only the set of candidates matters here
-    const float3 v01 = vtx(0, 1), v10 = vtx(1, 0);
+    float2 tvk = make_float2(0.f, 0.f);
+    float3 v00, v01, v10, v11;
+    if (KEPT || wi != 0xffffffffu) {
+        const float* p = kept_quad(ws, wi, i, j);
+        v00 = load3(p); v01 = load3(p + 3);
+        v10 = load3(p + 3 * (kBinQX + 1)); v11 = load3(p + 3 * (kBinQX + 1) + 3);
+        tvk = kept_validity(ws, wi, i, j);
+    } else {
+        float3 v[4];
+        eval_corners<4>(g, i, j, 0xcu, 0xau, v, &und);
+        v00 = v[0]; v01 = v[1]; v10 = v[2]; v11 = v[3];
+    }
     const bool gate = v01.z > 0.f && v10.z > 0.f && v01.x > 0.f && v10.x > 0.f;
     const uint32_t s0 = e << 2;
-    {
-        const float3 v00 = vtx(0, 0);
-        if (gate && v00.z > 0.f && v00.x > 0.f)
-            raster_tri<TILE>(v00, v01, v10, s0, false, tx0, ty0, out_w, out_h, g.rescale, key1, key2, und,
-                             tvk.x, Q);
-    }
-    {
-        const float3 v11 = vtx(1, 1);
-        if (gate && v11.z > 0.f && v11.x > 0.f)
-            raster_tri<TILE>(v11, v10, v01, s0 | 1u, false, tx0, ty0, out_w, out_h, g.rescale, key1, key2, und,
-                             tvk.y, Q);
-    }
-    if (gate && g.wrap && j == 0) {
-        const float3 v00 = vtx(0, 0);
-        const float3 l0 = vertex(g, i, g.sw - 1, &und), l1 = vertex(g, i + 1, g.sw - 1, &und);
-        raster_tri<TILE>(l0, v00, l1, s0 | 2u, true, tx0, ty0, out_w, out_h, g.rescale, key1, key2, und, 0.f,
-                         (Queue*)nullptr);
-        raster_tri<TILE>(v10, l1, v00, s0 | 3u, true, tx0, ty0, out_w, out_h, g.rescale, key1, key2, und, 0.f,
-                         (Queue*)nullptr);
+    if (gate && v00.z > 0.f && v00.x > 0.f)
+        raster_tri<TILE, KEPT>(v00, v01, v10, s0, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und, tvk.x, Q);
+    if (gate && v11.z > 0.f && v11.x > 0.f)
+        raster_tri<TILE, KEPT>(v11, v10, v01, s0 | 1u, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und,
+                               tvk.y, Q);
+    if (__builtin_expect(gate && gt.wrap && j == 0, 0)) {
+        float3 l[2];
+        if (KEPT) kept_seam(ws, d, vs, i, g.sw, l);
+        else eval_corners<2>(g, i, g.sw - 1, 2u, 0u, l, &und);
+#pragma unroll 1
+        for (uint32_t k = 0; k < 2u; ++k) {
+            const bool s3 = k != 0u;
+            raster_tri<TILE, false>(s3 ? v10 : l[0], s3 ? l[1] : v00, s3 ? v00 : l[1], s0 | (2u + k), true, tx0, ty0,
+                                    out_w, out_h, gt.rescale, key1, key2, und, 0.f, (Queue*)nullptr);
+        }
     }
     if (C) {
         C->ij[e] = ij;
@@ -1194,29 +1236,50 @@ __device__ inline void encode_tile_pixel(const ViewDesc& vd, float3 c, int px, i
     }
 }
 
-// MULTI: more sources than one phase holds (the phases loop, and the blend
-// state lives across them); otherwise one phase, which keeps the coverage pass
-// free of the blend state's registers.
-// TILE: the tile edge; a block has a thread per pixel (256 or 1024 threads),
-// and the caches scale with the tile's area.
-template <class G, int MODE, bool MULTI, int TILE>
-__global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_eu(MULTI ? (TILE > kTile ? 4 : 6) : 8))) k_raster(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
-                                                BatchDims d, RasterWS ws) {
-    constexpr int NT = TILE * TILE;
-    constexpr int AREA = NT / (kTile * kTile);
-    constexpr int GRP = MULTI ? kRasterGroupMulti : kRasterGroup;   // sources per phase
-    __shared__ unsigned long long key1[GRP][NT];
-    __shared__ uint32_t key2[GRP][NT];
-    __shared__ uint32_t pref[GRP + 1];
-    __shared__ uint32_t boff[GRP];   // list offsets of the phase's bins
-    __shared__ int s_deferred;   // any pixel of the tile deferred
-    __shared__ int s_hole;       // any pixel of the tile a hole (quality not > 0)
+// LDS of a k_raster block.
+template <bool MULTI, int TILE>
+struct RasterLds {
+    static constexpr int NT = TILE * TILE;
+    static constexpr int AREA = NT / (kTile * kTile);
+    static constexpr int GRP = MULTI ? kRasterGroupMulti : kRasterGroup;   // sources per phase
+    unsigned long long key1[GRP][NT];
+    uint32_t key2[GRP][NT];
+    uint32_t pref[GRP + 1];
+    uint32_t boff[GRP];   // list offsets of the phase's bins
+    int s_deferred;       // any pixel of the tile deferred
+    int s_hole;           // any pixel of the tile a hole (quality not > 0)
     // one phase: a smaller cache keeps a 16 x 16 block within 20 KB of LDS (8 blocks per CU)
-    __shared__ RasterCache<(MULTI ? kRasterCache : kRasterCacheOne) * AREA> cache;
+    RasterCache<(MULTI ? kRasterCache : kRasterCacheOne) * AREA> cache;
     typedef WideQueue<(MULTI ? kWideQueue : kWideQueueOne) * AREA> Queue;
-    __shared__ Queue wide;
+    Queue wide;
+};
+
+// One tile of k_raster.  Bound by the issue of VALU instructions (0.62 T/s of wave
+// instructions; 1024 SIMDs issue 0.61 T/s at 2.4 GHz).  Raster ms with the box and the narrowing one
+// after the other, the candidates marked by exact numerators and every
+// barycentric divided out, vertex code in one body -> now: 16 views of mixed
+// sizes 3.13 -> 2.57, one 1920x1080 view 0.246 -> 0.194 (four 4096x2048
+// panoramas); 8192x4096 panorama of eleven 11.0 -> 7.9; two 3840x2160 views of
+// 11 perspective sources 3.42 -> 2.87.  KEPT: every surviving work item keeps its vertex
+// window and validities (nearly always), so this code evaluates no vertex and
+// no validity of slots 0 and 1: a third of the instructions of the general
+// form, whose registers would otherwise spill around them.
+template <class G, int MODE, bool MULTI, int TILE, bool KEPT>
+__device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
+                                            const BatchDims& d, const RasterWS& ws, RasterLds<MULTI, TILE>& L) {
+    typedef RasterLds<MULTI, TILE> Lds;
+    typedef typename Lds::Queue Queue;
+    constexpr int NT = Lds::NT, GRP = Lds::GRP;
+    auto& key1 = L.key1;
+    auto& key2 = L.key2;
+    auto& pref = L.pref;
+    auto& boff = L.boff;
+    auto& cache = L.cache;
+    Queue& wide = L.wide;
+    int& s_deferred = L.s_deferred;
+    int& s_hole = L.s_hole;
     const uint32_t T = tile_of_block(blockIdx.x, d.ntiles);
-    if (T >= d.ntiles || ws.status[1]) return;   // bins not filled: capacity reported to the host
+    if (T >= d.ntiles) return;
     const int v = find_view(views, d.nviews, T);
     const ViewDesc& vd = views[v];
     const int tile = (int)(T - vd.tile_base);
@@ -1268,13 +1331,13 @@ __global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_e
             int k = 0;
             while (k + 1 < gs && e >= pref[k + 1]) ++k;
             const uint32_t ij = ws.lists[(size_t)boff[k] + (e - pref[k])];
-            raster_quad<TILE>(gv[s0 + k], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k], cached ? &cache : nullptr,
+            raster_quad<TILE, KEPT>(gv[s0 + k], gv[0], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k], cached ? &cache : nullptr,
                               &wide, ws, d, (uint32_t)(v * d.nsrc + s0 + k));
         }
         __syncthreads();
         const uint32_t nwide = __builtin_amdgcn_readfirstlane(min(wide.n, Queue::cap));
         if (nwide) {   // the same in every wave
-            raster_wide<TILE, NT>(gv + s0, boff, pref, gs, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1,
+            raster_wide<TILE, NT, KEPT>(gv + s0, boff, pref, gs, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1,
                                   key2, ws, d, (uint32_t)(v * d.nsrc + s0));
             __syncthreads();
         }
@@ -1299,32 +1362,35 @@ __global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_e
                     const uint32_t id = (uint32_t)kw, e = id >> 2;
                     const int slot = (int)(id & 3u);
                     const G& g = gv[s];
+                    const uint32_t vs = (uint32_t)(v * d.nsrc + s);
+                    const uint32_t ij = cached ? cache.ij[e] : ws.lists[(size_t)boff[k] + (e - pref[k])];
                     int i, j;
-                    const float* vb = nullptr;
-                    uint32_t wk = 0xffffffffu;
-                    if (cached) {
-                        unpack_ij(cache.ij[e], i, j);
-                        if (slot < 2) wk = cache.wi[e];
-                        if (wk != 0xffffffffu) vb = ws.vbuf + (size_t)wk * (3 * kBinVerts);
-                    }
-                    if (vb) {
+                    unpack_ij(ij, i, j);
+                    const uint32_t wk = cached ? cache.wi[e] : kept_index<KEPT>(ws, d, vs, i, j);
+                    bool ok = true;
+                    if (slot < 2 && (KEPT || wk != 0xffffffffu)) {
                         // T1: v00 v01 v10; T2: v11 v10 v01 (corner offsets of slot_vertex);
                         // the validity the counting pass kept (the coverage pass used it)
-                        const int li = i % kBinQY, lj = j % kBinQX;
-                        const float3 a = kept_vertex(vb, li + slot, lj + slot);
-                        const float3 b = kept_vertex(vb, li + slot, lj + 1 - slot);
-                        const float3 cc = kept_vertex(vb, li + 1 - slot, lj + slot);
+                        const float* p = kept_quad(ws, wk, i, j);
+                        const float3 a = load3(p + (slot ? 3 * (kBinQX + 2) : 0));
+                        const float3 b = load3(p + (slot ? 3 * (kBinQX + 1) : 3));
+                        const float3 cc = load3(p + (slot ? 3 : 3 * (kBinQX + 1)));
                         const float2 tvk = kept_validity(ws, wk, i, j);
                         resolve_cached(g, i, j, slot, a, b, cc, slot ? tvk.y : tvk.x, px, py, c, dep, shape);
+                    } else if (KEPT) {   // slot 2: l0 v00 l1, slot 3: v10 l1 v00
+                        const float* p = kept_quad(ws, wk, i, j);
+                        const float3 v00 = load3(p), v10 = load3(p + 3 * (kBinQX + 1));
+                        float3 l[2];
+                        kept_seam(ws, d, vs, i, g.sw, l);
+                        const float3 a = slot == 2 ? l[0] : v10, b = slot == 2 ? v00 : l[1], cc = slot == 2 ? l[1] : v00;
+                        Tri T;
+                        tri_load(T, a, b, cc);
+                        ok = tri_validity_fast(T, g.rescale, T.tv);
+                        resolve_cached(g, i, j, slot, a, b, cc, T.tv, px, py, c, dep, shape);
                     } else {
-                        const uint32_t ij = cached ? cache.ij[e] : ws.lists[(size_t)boff[k] + (e - pref[k])];
-                        unpack_ij(ij, i, j);
-                        if (!resolve<true>(g, i, j, slot, px, py, c, dep, shape, vd.w, vd.h,
-                                           kept_block(ws, d, (uint32_t)(v * d.nsrc + s), i, j))) {
-                            deferred = true;
-                            break;
-                        }
+                        ok = resolve<true>(g, i, j, slot, px, py, c, dep, shape, vd.w, vd.h, kept_block(ws, d, vs, i, j));
                     }
+                    if (!ok) { deferred = true; break; }
                 }
                 if (MODE == MODE_RAW) {
                     rc = c; rd = dep; rs = shape;
@@ -1366,6 +1432,22 @@ __global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_e
             ws.deferred_tiles[k] = T;
         }
     }
+}
+
+// MULTI: more sources than one phase holds (the phases loop, and the blend
+// state lives across them); otherwise one phase, which keeps the coverage pass
+// free of the blend state's registers.
+// TILE: the tile edge; a block has a thread per pixel (256 or 1024 threads),
+// and the caches scale with the tile's area.
+template <class G, int MODE, bool MULTI, int TILE>
+__global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_eu(MULTI ? (TILE > kTile ? 4 : 6) : 8)))
+k_raster(const G* __restrict__ geoms, const ViewDesc* __restrict__ views, BatchDims d, RasterWS ws) {
+    __shared__ RasterLds<MULTI, TILE> lds;
+    if (ws.status[1]) return;   // bins not filled: capacity reported to the host
+    if (d.kept_geom && ws.status[4] <= d.range_cap)   // the same for the whole launch
+        raster_tile<G, MODE, MULTI, TILE, true>(geoms, views, d, ws, lds);
+    else
+        raster_tile<G, MODE, MULTI, TILE, false>(geoms, views, d, ws, lds);
 }
 
 // ------------------------------------------------------ in-order replay
