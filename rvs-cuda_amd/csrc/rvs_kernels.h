@@ -74,13 +74,13 @@ struct ViewDesc {
 
 // Device-side state of one launch set.
 struct RasterWS {
-    uint32_t* counts;        // [global tile][source] entries per bin (counting pass)
-    uint32_t* offsets;       // [global tile][source] first entry of each bin in lists
-    uint32_t* fill;          // [global tile][source] fill cursors
+    uint32_t* counts;        // [source][global tile] entries per bin
+    uint32_t* offsets;       // [source][global tile] first entry of each bin in lists
+    uint32_t* fill;          // [source][global tile] entries that the counting pass gave no place; then their cursors
     uint32_t* lists;         // [cap] quad codes (row << 16 | column), bins back to back
     uint32_t* ranges;        // [range_cap work items][256] packed tile range of each quad
-    uint2* ktab;             // [range_cap work items][1 + kBinTable]: the counting pass's LDS bin
-                             // table of the item, [0].x = n used slots, then n of (slot | count << 8, tile)
+    uint2* ktab;             // [range_cap work items][1 + kBinTable]: the bins of the counting pass's LDS
+                             // table of the item, [0].x = n, then n of (first of its places in the bin, tile)
     float* vbuf;             // [range_cap work items][kBinQY + 1][kBinQX + 1][3] vertices (u', v', depth)
     float2* tvq;             // [range_cap work items][256] validity of triangles T1, T2 of each quad
     uint32_t* imap;          // [view][source][item] work index of a kept item, ~0 otherwise

@@ -99,6 +99,10 @@ __device__ inline uint32_t tile_of_block(uint32_t b, uint32_t ntiles) {
     return (b % 8) * per + b / 8;
 }
 
+// Bin of source s in global tile t.  Bins of one source are adjacent along a
+// tile row, so that the atomics of a quad across many tiles share cache lines.
+__device__ inline size_t bin_index(const BatchDims& d, uint32_t t, uint32_t s) { return (size_t)s * d.ntiles + t; }
+
 // ------------------------------------------------------------------ quads
 
 // vertex() of the N corners (i + di, j + dj), bit k of ROWS / COLS being di /
@@ -364,21 +368,27 @@ __global__ void __launch_bounds__(kCullThreads) k_bin_cull(const G* __restrict__
 // Bins are compact: a counting pass (k_bin<COUNT>) finds every surviving
 // quad's tile range and counts the (quad, tile) entries per (tile, source)
 // bin; an exclusive scan turns the counts into bin offsets; fill passes write
-// the quad codes, taking slots through one fill cursor per bin.  For the first
-// range_cap work items the counting pass keeps each quad's tile range (and the
-// item's vertex window and triangle validities, for the raster), so their fill
-// pass (k_fill_kept) needs no vertex work; later items re-evaluate their
-// vertices in their fill pass (k_bin<FILL>).  The order of a bin's entries is
-// free: the raster's keys commute and the in-order replay sorts them.  When
-// the entries exceed the list capacity the fill passes and the raster are
-// skipped and the needed capacity is reported.
+// the quad codes.  For the first range_cap work items the counting pass keeps
+// each quad's tile range (and the item's vertex window and triangle
+// validities, for the raster) and reserves the item's places in its bins, so
+// their fill pass (k_fill_kept) needs neither vertex work nor atomics on
+// memory; later items re-evaluate their vertices in their fill pass
+// (k_bin<FILL>) and take places through one cursor per bin, behind the reserved
+// ones.  The order of a bin's entries is free: the raster's keys commute and
+// the in-order replay sorts them.  When the entries exceed the list capacity
+// the fill passes and the raster are skipped and the needed capacity is
+// reported.
 //
 // Blocks first gather their entries per bin in an LDS table (a few to a few
 // dozen distinct tiles per 64x4 quad block), then take one global atomic per
 // bin: device-scope atomics are performed at the memory side, so their number
-// and the chains of dependent ones set these kernels' time.  The counting
-// pass needs no atomic's return value (its atomics do not hold the block);
-// the fill passes take one returning atomic per bin.
+// and the cache lines they touch cost the wide-range scenes most of their
+// binning time.
+//
+// The counting pass is bound by VALU issue (0.55 of 0.61 T wave instructions/s).  Of its
+// 995 us for 16 mixed views before the validity's shorter form: vertices 290,
+// validities 270, boxes 200, stores of the kept state 130, tile walk 123,
+// count atomics 0 (builds that skip a part).
 
 constexpr uint32_t kRangeNone = 0xffffffffu;   // no surviving triangle
 constexpr uint32_t kRangeBig = 0xfffffffeu;    // range too wide to pack: re-evaluated
@@ -468,23 +478,6 @@ __device__ inline int find_slot(const uint32_t* keys, uint32_t t) {
     return -1;
 }
 
-// Tile range [tx0, tx1] x [ty0, ty1] touched by the narrowed bounding boxes
-// of a quad's surviving triangles; false when none can cover a pixel.
-__device__ inline bool quad_tiles(Quad& Q, int out_w, int out_h, int shift, int& tx0, int& tx1, int& ty0, int& ty1) {
-    if (!Q.alive) return false;
-    int xmin = INT_MAX, xmax = INT_MIN, ymin = INT_MAX, ymax = INT_MIN;
-    for (int k = 0; k < 4; ++k)
-        if (Q.alive & (1u << k)) {
-            int xa, xb, ya, yb;   // as quad_range_tv: the pixels it can cover
-            if (!tri_box(Q.t[k], out_w, out_h, 0, out_w - 1, 0, out_h - 1, xa, xb, ya, yb)) continue;
-            xmin = min(xmin, xa); xmax = max(xmax, xb);
-            ymin = min(ymin, ya); ymax = max(ymax, yb);
-        }
-    if (xmin > xmax) return false;
-    tx0 = xmin >> shift; tx1 = xmax >> shift; ty0 = ymin >> shift; ty1 = ymax >> shift;
-    return true;
-}
-
 // Block-cooperative walk over the tiles of the threads' quad ranges: entry e
 // of the block's concatenated ranges goes to thread e % 256, which finds the
 // owning quad by a binary search of the block-wide inclusive scan of the
@@ -501,6 +494,15 @@ struct RangeWalk {
 };
 
 constexpr uint32_t kLaneTiles = 4;   // ranges up to this many tiles stay with their own lane
+// Ranges above this many tiles (quads across the seam or near a pole of an
+// equirectangular target, up to a whole row of tiles or more) would fill the
+// table and then probe it in vain: their entries take a place each from their
+// bins' cursors, a lane per tile, neighbouring tiles in neighbouring lanes.
+// Below it the table saves atomics where several quads of an item share tiles.
+// Counting pass plus fill, with bins of one tile adjacent and every entry
+// tried in the table -> now: a 1920x1080 view beside a pole of its sources 0.60
+// -> 0.19 ms, an 8192x4096 panorama of eleven with close objects 10.9 -> 4.2 ms.
+constexpr uint32_t kTableTiles = 64;
 
 // Publishes this thread's range (n = 0: none); all 256 threads call it, and
 // the walk may start after the __syncthreads() that follows.
@@ -531,7 +533,8 @@ __device__ inline void range_walk(const RangeWalk& W, int tid, F fn) {
         }
         const uint32_t l = e - (lo ? W.incl[lo - 1] : 0u);
         const uint32_t o = W.org[lo], w = W.wid[lo];
-        fn(lo, (int)(o & 0xffffu) + (int)(l % w), (int)(o >> 16) + (int)(l / w));
+        fn(lo, (int)(o & 0xffffu) + (int)(l % w), (int)(o >> 16) + (int)(l / w),
+           W.incl[lo] - (lo ? W.incl[lo - 1] : 0u) <= kTableTiles);
     }
 }
 
@@ -596,7 +599,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
             }
         }
         auto tile_of = [&](int tx, int ty) { return vd.tile_base + (uint32_t)(ty * vd.tiles_x + tx); };
-        auto bin_of = [&](uint32_t t) { return (size_t)t * d.nsrc + s; };
+        auto bin_of = [&](uint32_t t) { return bin_index(d, t, (uint32_t)s); };
         // the range of a kept quad, for its fill pass
         if (!FILL && stored)
             ws.ranges[(size_t)wi * 256 + tid] = more ? pack_range(tx0, tx1, ty0, ty1) : kRangeNone;
@@ -613,42 +616,43 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
         auto each_tile = [&](auto fn) {
             if (more && !wide)
                 for (int ty = ty0; ty <= ty1; ++ty)
-                    for (int tx = tx0; tx <= tx1; ++tx) fn(tid, tx, ty);
+                    for (int tx = tx0; tx <= tx1; ++tx) fn(tid, tx, ty, true);
             if (any_wide) range_walk(walk, tid, fn);
         };
-        each_tile([&](int lane, int tx, int ty) {
+        each_tile([&](int lane, int tx, int ty, bool table) {
             const uint32_t t = tile_of(tx, ty);
-            const int k = table_slot(t_key, t);
+            const int k = table ? table_slot(t_key, t) : -1;
             if (k >= 0) {
                 atomicAdd(&t_n[k], 1u);
-            } else if (FILL) {   // table full: a slot of its own
+            } else if (FILL) {   // not in the table: a place of its own
                 const size_t bin = bin_of(t);
                 ws.lists[(size_t)ws.offsets[bin] + atomicAdd(&ws.fill[bin], 1u)] = quad_of(lane);
             } else {
-                atomicAdd(&ws.counts[bin_of(t)], 1u);
+                atomicAdd(&ws.fill[bin_of(t)], 1u);
             }
         });
         __syncthreads();   // table complete
+        uint32_t rank = 0u;
         if (tid < kBinTable && t_n[tid]) {
             const size_t bin = bin_of(t_key[tid]);
             if (FILL) t_base[tid] = ws.offsets[bin] + atomicAdd(&ws.fill[bin], t_n[tid]);
-            else atomicAdd(&ws.counts[bin], t_n[tid]);
+            else if (stored) rank = atomicAdd(&ws.counts[bin], t_n[tid]);
+            else atomicAdd(&ws.fill[bin], t_n[tid]);
         }
         if (stored) {
-            // the item's table for its fill pass: the used slots (slot, count,
-            // tile) in any order, their number first
+            // the item's table for its fill pass: (rank, tile) of the used slots
+            // in any order, their number first
             if (tid == 0) t_used = 0u;
             __syncthreads();
             uint2* kt = ws.ktab + (size_t)wi * (1 + kBinTable);
-            if (tid < kBinTable && t_n[tid])
-                kt[1 + atomicAdd(&t_used, 1u)] = make_uint2((uint32_t)tid | (t_n[tid] << 8), t_key[tid]);
+            if (tid < kBinTable && t_n[tid]) kt[1 + atomicAdd(&t_used, 1u)] = make_uint2(rank, t_key[tid]);
             __syncthreads();
             if (tid == 0) kt[0] = make_uint2(t_used, 0u);
         }
         if (FILL) {
             __syncthreads();   // bases known
-            each_tile([&](int lane, int tx, int ty) {
-                const int k = find_slot(t_key, tile_of(tx, ty));
+            each_tile([&](int lane, int tx, int ty, bool table) {
+                const int k = table ? find_slot(t_key, tile_of(tx, ty)) : -1;
                 if (k >= 0) ws.lists[atomicAdd(&t_base[k], 1u)] = quad_of(lane);
             });
         }
@@ -656,93 +660,129 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
     }
 }
 
-// Fill pass over the kept work items, a block per item (striding when there
-// are more items than blocks) and a thread per quad: entries take slots
-// through the item's LDS bin table, rebuilt from what the counting pass
-// stored, and one fill-cursor atomic per bin.  A quad whose range was too
-// wide to pack is re-binned from the kept vertices.
+// A quad of the fill pass with more than kLaneTiles tiles.
+struct WideFill {
+    uint32_t org;    // tx0 | ty0 << 16
+    uint32_t dim;    // tiles per row | rows << 16; 0: not known yet
+    uint32_t quad;
+};
+
+// Fill pass over the kept work items, a wave per item and four quads per lane:
+// the item's bins and the places reserved in them by the counting pass go to
+// an LDS table, from which every (quad, tile) entry takes its place.  Quads
+// with wide ranges are shared by the block's waves, a wave each with a lane
+// per tile (an item near a pole deals thousands of tiles).  A tile that found
+// the table full while counting takes its place from the bin's cursor.
+// Bound by latency: a chain of four dependent accesses per item, so items in
+// flight matter most.  Against a block per item with a returning cursor atomic
+// per bin (six accesses in the chain, 8 items per CU instead of 32): 16 mixed
+// views 455 -> 280 us, an 8192x4096 panorama of eleven 1.4 -> 1.2 ms.
 template <class G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k_fill_kept(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
                                                    BatchDims d, RasterWS ws) {
-    __shared__ uint32_t t_key[kBinTable];
-    __shared__ uint32_t t_base[kBinTable];
-    __shared__ RangeWalk walk;
+    __shared__ uint32_t t_key[4][kBinTable];
+    __shared__ uint32_t t_base[4][kBinTable];
+    __shared__ WideFill wide[4][256];   // [wave whose item it is]
+    __shared__ uint32_t nwide[4];
+    __shared__ uint32_t w_vs[4];        // (view, source) of the waves' items
     if (ws.status[1]) return;   // list capacity exceeded: nothing to fill
-    const uint32_t lim = min(ws.status[4], d.range_cap);
-    const int tid = threadIdx.x;
+    const uint64_t lim = min(ws.status[4], d.range_cap);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t per = d.bins_x * d.bins_y;
-    for (uint32_t wi = blockIdx.x; wi < lim; wi += gridDim.x) {
-        if (tid < kBinTable) t_key[tid] = kTableEmpty;
-        const uint32_t code = ws.work[wi];
-        const uint32_t item = code % per, vs = code / per;
-        const int s = (int)(vs % (uint32_t)d.nsrc), v = (int)(vs / (uint32_t)d.nsrc);
-        const ViewDesc& vd = views[v];
-        const int i0 = (int)(item / d.bins_x) * kBinQY, j0 = (int)(item % d.bins_x) * kBinQX;
-        const int i = i0 + tid / kBinQX, j = j0 + tid % kBinQX;
-        const uint32_t r = ws.ranges[(size_t)wi * 256 + tid];
-        bool more = false;
-        int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;
-        if (r == kRangeBig) {
-            const G& g = geoms[vs];
-            const float* vb = d.kept_geom ? ws.vbuf + (size_t)wi * (3 * kBinVerts) : nullptr;
-            Quad Q;
-            quad_build(Q, g, i, j,
-                       [&](int ii, int jj) -> float3 {
-                           const int rr = ii - i0, c = jj - j0;
-                           if (vb && rr >= 0 && rr <= kBinQY && c >= 0 && c <= kBinQX) return kept_vertex(vb, rr, c);
-                           return vertex(g, ii, jj);
-                       },
-                       vd.w, vd.h, false);
-            more = quad_tiles(Q, vd.w, vd.h, d.tile_shift, tx0, tx1, ty0, ty1);
-        } else if (r != kRangeNone) {
-            unpack_range(r, tx0, tx1, ty0, ty1);
-            more = true;
+    auto place = [&](int w, uint32_t t, uint32_t s, uint32_t quad, bool table) {
+        const int k = table ? find_slot(t_key[w], t) : -1;
+        if (k >= 0) {
+            ws.lists[atomicAdd(&t_base[w][k], 1u)] = quad;
+        } else {
+            const size_t bin = bin_index(d, t, s);
+            ws.lists[(size_t)ws.offsets[bin] + atomicAdd(&ws.fill[bin], 1u)] = quad;
         }
-        // entries (narrow ranges by their own lane, wide ones dealt to the
-        // block): LDS bin table, one fill-cursor atomic per bin
-        auto tile_of = [&](int tx, int ty) { return vd.tile_base + (uint32_t)(ty * vd.tiles_x + tx); };
-        auto quad_of = [&](int lane) {
-            return ((uint32_t)(i0 + lane / kBinQX) << 16) | (uint32_t)(j0 + lane % kBinQX);
-        };
-        const bool wide = more && (uint32_t)(tx1 - tx0 + 1) * (uint32_t)(ty1 - ty0 + 1) > kLaneTiles;
-        const bool any_wide = __syncthreads_or(wide);   // also orders the table clear
-        if (any_wide) {
-            range_publish(walk, tid, wide, tx0, tx1, ty0, ty1);
-            __syncthreads();   // ranges scanned
-        }
-        auto each_tile = [&](auto fn) {
-            if (more && !wide)
-                for (int ty = ty0; ty <= ty1; ++ty)
-                    for (int tx = tx0; tx <= tx1; ++tx) fn(tid, tx, ty);
-            if (any_wide) range_walk(walk, tid, fn);
-        };
-        // the counting pass's table of this item, at the same slots (so
-        // find_slot sees the same probe sequences), with one fill-cursor
-        // atomic per used slot; a tile that found the table full there is
-        // absent here too and takes a slot of its own per entry
-        {
+    };
+    // item of wave w in a block's round: neighbouring items (those near a pole
+    // are all costly) go to different blocks
+    for (uint64_t b0 = blockIdx.x; b0 < lim; b0 += (uint64_t)gridDim.x * 4u) {
+        const uint64_t wi64 = b0 + (uint64_t)wave * gridDim.x;
+        const uint32_t wi = (uint32_t)wi64;
+        t_key[wave][lane] = kTableEmpty;
+        t_key[wave][lane + 64] = kTableEmpty;
+        if (lane == 0) nwide[wave] = 0u;
+        __syncthreads();
+        if (wi64 < lim) {   // the same for the wave
             const uint2* kt = ws.ktab + (size_t)wi * (1 + kBinTable);
+            const uint2 e0 = kt[1 + lane];   // with the count: entries past it are not used
+            uint32_t r[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = ws.ranges[(size_t)wi * 256 + q * 64 + lane];
             const uint32_t nused = kt[0].x;
-            if (tid < (int)nused) {
-                const uint2 e = kt[1 + tid];
-                const uint32_t slot = e.x & 0xffu, n = e.x >> 8;
-                t_key[slot] = e.y;
-                const size_t bin = (size_t)e.y * d.nsrc + s;
-                t_base[slot] = ws.offsets[bin] + atomicAdd(&ws.fill[bin], n);
+            const uint32_t code = ws.work[wi];
+            const uint32_t item = code % per, vs = code / per;
+            const uint32_t s = vs % (uint32_t)d.nsrc, v = vs / (uint32_t)d.nsrc;
+            const ViewDesc& vd = views[v];
+            const int i0 = (int)(item / d.bins_x) * kBinQY, j0 = (int)(item % d.bins_x) * kBinQX;
+            if (lane == 0) w_vs[wave] = vs;
+            auto take = [&](uint2 e) {
+                const uint32_t base = ws.offsets[bin_index(d, e.y, s)] + e.x;
+                t_base[wave][table_slot(t_key[wave], e.y)] = base;   // at most kBinTable tiles: never full
+            };
+            if (lane < (int)nused) take(e0);
+            if (lane + 64 < (int)nused) take(kt[65 + lane]);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (r[q] == kRangeNone) continue;
+                int tx0, tx1, ty0, ty1;
+                unpack_range(r[q], tx0, tx1, ty0, ty1);
+                const uint32_t quad = ((uint32_t)(i0 + q) << 16) | (uint32_t)(j0 + lane);
+                const uint32_t nx = (uint32_t)(tx1 - tx0 + 1), ny = (uint32_t)(ty1 - ty0 + 1);
+                if (r[q] == kRangeBig || nx * ny > kLaneTiles) {
+                    WideFill& w = wide[wave][atomicAdd(&nwide[wave], 1u)];
+                    w.org = (uint32_t)tx0 | ((uint32_t)ty0 << 16);
+                    w.dim = r[q] == kRangeBig ? 0u : nx | (ny << 16);
+                    w.quad = quad;
+                    continue;
+                }
+                for (int ty = ty0; ty <= ty1; ++ty)
+                    for (int tx = tx0; tx <= tx1; ++tx)
+                        place(wave, vd.tile_base + (uint32_t)(ty * vd.tiles_x + tx), s, quad, true);
             }
         }
-        __syncthreads();   // table and bases known
-        each_tile([&](int lane, int tx, int ty) {
-            const uint32_t t = tile_of(tx, ty);
-            const int k = find_slot(t_key, t);
-            if (k >= 0) {
-                ws.lists[atomicAdd(&t_base[k], 1u)] = quad_of(lane);
-            } else {
-                const size_t bin = (size_t)t * d.nsrc + s;
-                ws.lists[(size_t)ws.offsets[bin] + atomicAdd(&ws.fill[bin], 1u)] = quad_of(lane);
+        __syncthreads();   // wide quads known
+        for (int o = 0; o < 4; ++o) {
+            const uint32_t nw = nwide[o];
+            if (nw == 0u) continue;
+            const uint32_t vs = __builtin_amdgcn_readfirstlane(w_vs[o]);
+            const uint32_t s = vs % (uint32_t)d.nsrc;
+            const ViewDesc& vd = views[vs / (uint32_t)d.nsrc];
+            for (uint32_t k = (uint32_t)wave; k < nw; k += 4u) {
+                const WideFill w = wide[o][k];
+                int tx0 = (int)(w.org & 0xffffu), ty0 = (int)(w.org >> 16);
+                uint32_t nx = w.dim & 0xffffu, ny = w.dim >> 16;
+                if (w.dim == 0u) {   // too wide to pack: binned again
+                    const G& g = geoms[vs];
+                    int i, j, tx1, ty1;
+                    unpack_ij(w.quad, i, j);
+                    float3 c[4];
+                    if (d.kept_geom) {
+                        const float* p = kept_quad(ws, (uint32_t)b0 + (uint32_t)o * gridDim.x, i, j);
+                        c[0] = load3(p); c[1] = load3(p + 3);
+                        c[2] = load3(p + 3 * (kBinQX + 1)); c[3] = load3(p + 3 * (kBinQX + 1) + 3);
+                    } else {
+                        eval_corners<4>(g, i, j, 0xcu, 0xau, c, nullptr);
+                    }
+                    if (!quad_range_tv(g, i, j, c[0], c[1], c[2], c[3], vd.w, vd.h, d.tile_shift, tx0, tx1, ty0, ty1,
+                                       nullptr))
+                        continue;
+                    nx = (uint32_t)(tx1 - tx0 + 1);
+                    ny = (uint32_t)(ty1 - ty0 + 1);
+                }
+                for (uint32_t e = (uint32_t)lane; e < nx * ny; e += 64u)
+                    place(o, vd.tile_base + ((uint32_t)ty0 + e / nx) * (uint32_t)vd.tiles_x + (uint32_t)tx0 + e % nx, s,
+                          w.quad, nx * ny <= kTableTiles);
             }
-        });
-        __syncthreads();   // table free for the next item
+        }
+        __syncthreads();   // LDS free for the next items
     }
 }
 
@@ -751,15 +791,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
 // it exceeds the list capacity).
 constexpr int kScanPer = 2048;   // bins per scan block (256 threads x 8)
 
-__global__ void __launch_bounds__(256) k_scan_blocks(const uint32_t* __restrict__ counts, uint32_t* offsets,
-                                                     size_t n, unsigned long long* bsum) {
+// A bin's entries are those with a place (counts) and, behind them, those
+// without (fill); counts becomes their sum and fill the cursor of the latter.
+__global__ void __launch_bounds__(256) k_scan_blocks(uint32_t* counts, uint32_t* fill, uint32_t* offsets, size_t n,
+                                                     unsigned long long* bsum) {
     __shared__ unsigned long long part[256];
     const size_t base = (size_t)blockIdx.x * kScanPer + (size_t)threadIdx.x * 8;
     uint32_t c[8];
     unsigned long long sum = 0;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        c[k] = base + k < n ? counts[base + k] : 0u;
+        c[k] = 0u;
+        if (base + k < n) {
+            const uint32_t placed = counts[base + k], loose = fill[base + k];
+            c[k] = placed + loose;
+            if (loose) counts[base + k] = c[k];
+            fill[base + k] = placed;
+        }
         sum += c[k];
     }
     part[threadIdx.x] = sum;
@@ -840,12 +888,13 @@ hipError_t launch_bin(const G* geoms, const ViewDesc* views, const BatchDims& d,
         hipLaunchKernelGGL((k_bin<G, false, false>), dim3((unsigned)blocks), dim3(256), 0, s, geoms, views, d, ws);
     const size_t nbins = (size_t)d.ntiles * d.nsrc;
     const size_t nb = scan_blocks(nbins);
-    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nb), dim3(256), 0, s, ws.counts, ws.offsets, nbins, ws.bsum);
+    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nb), dim3(256), 0, s, ws.counts, ws.fill, ws.offsets, nbins,
+                       ws.bsum);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, ws.bsum, (uint32_t)nb, d.cap, ws.status);
     hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((nbins + 255) / 256)), dim3(256), 0, s, ws.offsets, nbins,
                        ws.bsum);
     if (d.range_cap)
-        hipLaunchKernelGGL(k_fill_kept<G>, dim3(flat), dim3(256), 0, s, geoms, views, d, ws);
+        hipLaunchKernelGGL(k_fill_kept<G>, dim3((flat + 3) / 4), dim3(256), 0, s, geoms, views, d, ws);
     if (total > d.range_cap)
         hipLaunchKernelGGL((k_bin<G, true, false>), dim3((unsigned)blocks), dim3(256), 0, s, geoms, views, d, ws);
     return hipGetLastError();
@@ -1306,7 +1355,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
             uint32_t cnt[GRP], off[GRP];
 #pragma unroll
             for (int k = 0; k < GRP; ++k) {
-                const size_t b = (size_t)T * d.nsrc + s0 + (k < gs ? k : 0);
+                const size_t b = bin_index(d, T, (uint32_t)(s0 + (k < gs ? k : 0)));
                 cnt[k] = ws.counts[b];
                 off[k] = ws.offsets[b];
             }
@@ -1695,7 +1744,7 @@ __global__ void __launch_bounds__(256) k_fallback(const G* __restrict__ geoms, c
         float rd = __builtin_inff(), rs = 0.f;
         for (int s = 0; s < d.nsrc; ++s) {
             const G& g = gv[s];
-            const size_t bin = (size_t)T * d.nsrc + s;
+            const size_t bin = bin_index(d, T, (uint32_t)s);
             const uint32_t n = ws.counts[bin];
             FoldState fs;
             replay_source(g, ws.lists + ws.offsets[bin], n, tx0, ty0, vd.w, vd.h, mine, px, py, dmask, sorted, rec,
@@ -1762,7 +1811,7 @@ __global__ void __launch_bounds__(256) k_fallback_src(const G* __restrict__ geom
             const bool mine = inside && ws.deferred[vd.px_base + o];
             dmask[tid] = mine ? 1 : 0;
             if (!__syncthreads_or(mine ? 1 : 0)) continue;
-            const size_t bin = (size_t)T * d.nsrc + s;
+            const size_t bin = bin_index(d, T, (uint32_t)s);
             FoldState fs;
             replay_source(g, ws.lists + ws.offsets[bin], ws.counts[bin], tx0, ty0, vd.w, vd.h, mine, px, py, dmask,
                           sorted, rec, pool_n, fs, ws, d, (uint32_t)(v * d.nsrc + s));
