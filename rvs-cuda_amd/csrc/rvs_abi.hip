@@ -135,7 +135,7 @@ struct Layout {
 // deferred-pixel flags, deferred-tile list and binning work list.
 struct RasterPlan {
     rvs_k::BatchDims d;
-    size_t status, counts, offsets, fill, lists, ranges, ktab, vbuf, tvq, imap, bsum, deferred, dtiles, work, tile_enc,
+    size_t status, counts, offsets, fill, lists, ranges, ktab, vbuf, imap, bsum, deferred, dtiles, work, tile_enc,
         rbuf;
 };
 
@@ -196,8 +196,7 @@ void plan_raster(Layout& L, RasterPlan& R, int nsrc, int nviews, uint32_t ntiles
     d.kept_geom = 1;
     if (const char* env = std::getenv("RVS_KEPT_GEOM")) d.kept_geom = std::strtol(env, nullptr, 10) != 0;
     const size_t kg = d.kept_geom ? d.range_cap : 0;
-    R.vbuf = L.take(kg * 3 * rvs_k::kBinVerts * sizeof(float));
-    R.tvq = L.take(kg * 256 * sizeof(float2));
+    R.vbuf = L.take(kg * rvs_k::kItemFloats * sizeof(float));
     R.imap = L.take((size_t)items * sizeof(uint32_t));
     R.deferred = L.take(npx);
     R.dtiles = L.take((size_t)ntiles * sizeof(uint32_t));
@@ -230,7 +229,6 @@ rvs_k::RasterWS carve_raster(char* base, const RasterPlan& R) {
     ws.ranges = (uint32_t*)(base + R.ranges);
     ws.ktab = (uint2*)(base + R.ktab);
     ws.vbuf = (float*)(base + R.vbuf);
-    ws.tvq = (float2*)(base + R.tvq);
     ws.imap = (uint32_t*)(base + R.imap);
     ws.deferred = (uint8_t*)(base + R.deferred);
     ws.deferred_tiles = (uint32_t*)(base + R.dtiles);
@@ -584,7 +582,7 @@ uint64_t noalloc_keep(const rvs_source* srcs, int n_src, const rvs_target* tgt, 
     need = P.total;
     if (P.total > kNoallocScratchBytes) return 0;
     const size_t per_item = 256 * sizeof(uint32_t) + (1 + rvs_k::kBinTable) * sizeof(uint2) +
-                            3 * (size_t)rvs_k::kBinVerts * sizeof(float) + 256 * sizeof(float2);
+                            (size_t)rvs_k::kItemFloats * sizeof(float);
     const uint64_t keep = 1 + (kNoallocScratchBytes - P.total) / per_item;
     // alignment of the four kept arrays can cost up to 4 x 255 bytes: step back until it fits
     for (uint64_t k = keep; k >= 1; k = k > 64 ? k - 64 : k - 1) {

@@ -246,22 +246,23 @@ __device__ inline float3 color(const PairGeom& g, int i, int j) {
     return make_float3(r.x * g.cscale, r.y * g.cscale, r.z * g.cscale);
 }
 
-// Colours of three source pixels (a triangle's corners), the same values as
-// three color() calls: the resident plane's three loads are issued together
-// and then converted, so that a resolve waits on memory once, not per corner.
-__device__ inline void color3(const PairGeom& g, const int r[3], const int c[3], float3 out[3]) {
+// Colours of three source pixels (a triangle's corners, linear indexes), the
+// same values as three color() calls: the resident plane's three loads are
+// issued together and then converted, so that a resolve waits on memory once,
+// not per corner.  The quarter goes into the scale, which is exact.
+__device__ inline void color3(const PairGeom& g, const uint32_t idx[3], float3 out[3]) {
     if (g.colq) {
         ushort4 q[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) q[k] = g.colq[(size_t)r[k] * g.sw + c[k]];
+        for (int k = 0; k < 3; ++k) q[k] = g.colq[idx[k]];
+        const float quarter = g.cscale * 0.25f;
 #pragma unroll
         for (int k = 0; k < 3; ++k)
-            out[k] = make_float3((float)q[k].x * g.cscale, ((float)q[k].y * 0.25f) * g.cscale,
-                                 ((float)q[k].z * 0.25f) * g.cscale);
+            out[k] = make_float3((float)q[k].x * g.cscale, (float)q[k].y * quarter, (float)q[k].z * quarter);
         return;
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) out[k] = color(g, r[k], c[k]);
+    for (int k = 0; k < 3; ++k) out[k] = color(g, (int)(idx[k] / (uint32_t)g.sw), (int)(idx[k] % (uint32_t)g.sw));
 }
 
 __device__ inline float3 color(const ArrayGeom& g, int i, int j) {
@@ -269,9 +270,12 @@ __device__ inline float3 color(const ArrayGeom& g, int i, int j) {
     return make_float3(g.color[3 * idx], g.color[3 * idx + 1], g.color[3 * idx + 2]);
 }
 
-__device__ inline void color3(const ArrayGeom& g, const int r[3], const int c[3], float3 out[3]) {
+__device__ inline void color3(const ArrayGeom& g, const uint32_t idx[3], float3 out[3]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) out[k] = color(g, r[k], c[k]);
+    for (int k = 0; k < 3; ++k) {
+        const float* p = g.color + 3 * (size_t)idx[k];
+        out[k] = make_float3(p[0], p[1], p[2]);
+    }
 }
 
 // ------------------------------------------------------------ triangles
@@ -406,7 +410,7 @@ __device__ inline bool tri_cover(const Tri& T, float n1, float n2, float& l1, fl
     return l1 >= -eps && l2 >= -eps && l3 >= -eps;
 }
 
-// The same with r = recip(den), den in quot_den's range.  Where a numerator is
+// The same with r = recip(den), den in cover_den's range.  Where a numerator is
 // outside quot_num's range l1 or l2 may differ from the division, but then it
 // is below 2^-20 either way, or the pixel is not covered either way.
 __device__ inline bool tri_cover_r(const Tri& T, float r, float n1, float n2, float& l1, float& l2, float& l3) {
@@ -538,6 +542,22 @@ __device__ inline void blend_step(BlendState& s, float3 c, float d, float shape,
         outMask = 0;
         if (q_acc > outQ) { out = s.c; outQ = q_acc; outMask = s.mask; }
         if (q_new > outQ) { out = c; outQ = q_new; outMask = m_new; }
+    } else if (s.mask != 0 && m_new) {
+        // both with a depth (in particular every uncovered view): only the
+        // second of the two sums below, without its branches
+        const bool u0 = q_acc > 0, u1 = q_new > 0;
+        const float w0 = rvs_pow(q_acc, a), w1 = rvs_pow(q_new, a);
+        float sum = 0.0f;
+        float3 inp = make_float3(0.f, 0.f, 0.f);
+        sum += u0 ? w0 : 0.f;
+        inp.x += u0 ? s.c.x * w0 : 0.f; inp.y += u0 ? s.c.y * w0 : 0.f; inp.z += u0 ? s.c.z * w0 : 0.f;
+        sum += u1 ? w1 : 0.f;
+        inp.x += u1 ? c.x * w1 : 0.f; inp.y += u1 ? c.y * w1 : 0.f; inp.z += u1 ? c.z * w1 : 0.f;
+        const bool none = sum == 0.0f;
+        const float r = 1.f / sum;
+        out = make_float3(none ? 0.f : inp.x * r, none ? 1.f : inp.y * r, none ? 0.f : inp.z * r);
+        outMask = 1;
+        outQ = none ? 0.f : rvs_pow(sum, a_inv);
     } else {
         float sumW = 0.0f, inpSum = 0.0f;
         float3 fin = make_float3(0.f, 0.f, 0.f), inp = make_float3(0.f, 0.f, 0.f);

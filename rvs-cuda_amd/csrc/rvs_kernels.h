@@ -28,6 +28,8 @@ constexpr int kFallbackSortCap = 8192;  // longest (source, tile) list the repla
                                         // ones are sorted in place in the entry list)
 constexpr int kMaxViews = 4096;
 constexpr int kBinVerts = (kBinQY + 1) * (kBinQX + 1);   // vertices of one binning work item
+constexpr int kItemTv = 2 * kBinQX * kBinQY;             // floats of a kept item: validities,
+constexpr int kItemFloats = kItemTv + 3 * kBinVerts;     // then vertices
 constexpr int kBinBlocks = 2048;    // persistent binning blocks (work items past the kept range)
 constexpr int kFlatBlocks = 65536;  // persistent blocks of the passes over the kept work items
 constexpr int kRasterGroup = 4;     // sources rasterised together in k_raster's one-phase instantiation
@@ -35,10 +37,10 @@ constexpr int kRasterGroupMulti = 4; // sources per phase of the looping instant
 constexpr int kRasterCache = 1536;  // binned quads per phase whose coverage-pass results stay in LDS
 constexpr int kRasterCacheOne = 960; // the same for launch sets of up to kRasterGroup sources (one phase)
 // k_raster: a triangle with more pixels of a tile than this in its box is shared by the lanes of a
-// wave.  8 views of 1920x1080 / one 8192x4096 equirectangular view, three scenes each, raster ms: 32 pixels
-// 1.17 1.92 1.07 / 12.4 15.3 13.8; 64: 1.22 1.82 1.10 / 10.9 15.8 12.6; 96: 1.27 1.84 1.11 / 10.8 16.1 12.4;
-// never: 1.80 3.00 1.30 / 10.7 18.1 12.2 (magnified triangles of one size fill whole waves near a
-// pole: side by side is as good there until they exceed a wave).
+// wave.  16 views of mixed sizes / an 8192x4096 equirectangular view, two scenes each, raster ms: 32
+// pixels 2.42 2.96 / 9.2 13.0; 64: 2.38 2.98 / 7.3 13.2; 96: 2.39 3.01 / 7.4 13.4; never, before the
+// other raster work: 18.1 for a view of 15.8 (magnified triangles of one size fill whole waves near
+// a pole: side by side is as good there until they exceed a wave).
 constexpr int kWidePx = 64;
 constexpr int kWideQueueOne = 100;  // such triangles put off per phase (in the LDS the one-phase blocks leave free)
 constexpr int kWideQueue = 500;     // the same in the looping instantiation
@@ -81,8 +83,8 @@ struct RasterWS {
     uint32_t* ranges;        // [range_cap work items][256] packed tile range of each quad
     uint2* ktab;             // [range_cap work items][1 + kBinTable]: the bins of the counting pass's LDS
                              // table of the item, [0].x = n, then n of (first of its places in the bin, tile)
-    float* vbuf;             // [range_cap work items][kBinQY + 1][kBinQX + 1][3] vertices (u', v', depth)
-    float2* tvq;             // [range_cap work items][256] validity of triangles T1, T2 of each quad
+    float* vbuf;             // [range_cap work items][kItemFloats]: validities of triangles T1, T2 of the
+                             // item's 256 quads, then its vertices [kBinQY + 1][kBinQX + 1][3] (u', v', depth)
     uint32_t* imap;          // [view][source][item] work index of a kept item, ~0 otherwise
     unsigned long long* bsum;// scan block sums
     uint8_t* deferred;       // [global pixel] pixel handled by the in-order replay
@@ -108,7 +110,7 @@ struct BatchDims {
                              // 5 (32 x 32, 1024-thread blocks)
     uint32_t flat_blocks;    // blocks of the passes over the kept work items
     uint32_t rbuf_tiles;     // deferred tiles whose sources are replayed in parallel (RasterWS::rbuf)
-    uint32_t kept_geom;      // kept work items also store vertex windows and validities (vbuf, tvq)
+    uint32_t kept_geom;      // kept work items also store vertex windows and validities (vbuf)
 };
 
 enum { MODE_BLEND = 0, MODE_RAW = 1 };

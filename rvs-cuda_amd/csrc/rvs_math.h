@@ -187,6 +187,10 @@ RVS_HD bool quot_num(float n) {   // [2^-50, 2^60]
     return a >= 8.881784197e-16f && a <= 1.152921505e18f;
 }
 
+// Denominators the raster's coverage test takes with recip: a quotient of at
+// most a few (anything larger is not covered) needs no tighter upper bound.
+RVS_HD bool cover_den(float d) { return d >= 9.313225746e-10f && d <= 1.208925820e24f; }   // [2^-30, 2^80]
+
 // Box [xa, xb] x [ya, yb] of the pixels in columns [x0, x1], rows [y0, y1]
 // that a triangle of positive denominator `den` can cover (empty when it can
 // cover none): pixel centres within 0.07 + 4e-6 s of its extent, s = largest

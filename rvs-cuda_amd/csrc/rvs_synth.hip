@@ -406,44 +406,57 @@ __device__ inline void unpack_range(uint32_t r, int& tx0, int& tx1, int& ty0, in
     ty1 = ty0 + (int)(r >> 28);
 }
 
-// Vertex (row lr, column lc) of a kept work item's vertex block (the counting
-// pass evaluated it with vertex(); the bits are the same).
 __device__ inline float3 load3(const float* p) { return make_float3(p[0], p[1], p[2]); }
+
+// Vertex window of kept work item wi (the counting pass evaluated it with
+// vertex(); the bits are the same).
+__device__ inline float* kept_window(const RasterWS& ws, uint32_t wi) {
+    return ws.vbuf + (size_t)wi * kItemFloats + kItemTv;
+}
 __device__ inline float3 kept_vertex(const float* vb, int lr, int lc) {
     return load3(vb + 3 * (lr * (kBinQX + 1) + lc));
 }
 
-// Work index of the kept work item holding quad (i, j) of pair vs, or ~0
-// (always ~0 when kept items store no vertex windows).  KEPT: every surviving
-// item is kept.
+// Work index of the kept work item holding quad ij of pair vs, or ~0 (always
+// ~0 when kept items store no vertex windows).  KEPT: every surviving item is
+// kept.  Fewer than 2^32 items, 2^14 item rows, 2^10 item columns.
+static_assert(kBinQX == 64 && kBinQY == 4 && kMaxSourceSide == 65536, "item of a quad code");
 template <bool KEPT = false>
-__device__ inline uint32_t kept_index(const RasterWS& ws, const BatchDims& d, uint32_t vs, int i, int j) {
+__device__ inline uint32_t kept_index(const RasterWS& ws, const BatchDims& d, uint32_t vs, uint32_t ij) {
     if (!KEPT && !d.kept_geom) return 0xffffffffu;
-    const uint32_t item = (uint32_t)(i / kBinQY) * d.bins_x + (uint32_t)(j / kBinQX);
-    return ws.imap[(size_t)vs * (d.bins_x * d.bins_y) + item];
+    return ws.imap[vs * (d.bins_x * d.bins_y) + __umul24(ij >> 18, d.bins_x) + ((ij >> 6) & 0x3ffu)];
 }
 
-// Upper left vertex of quad (i, j) in the window of kept item wi.
-__device__ inline const float* kept_quad(const RasterWS& ws, uint32_t wi, int i, int j) {
-    return ws.vbuf + (size_t)wi * (3 * kBinVerts) + 3 * ((i % kBinQY) * (kBinQX + 1) + j % kBinQX);
+// Place of quad ij in a kept item: its validities (T1, T2; the counting pass
+// evaluated them exactly, only alive triangles' values are meaningful) and its
+// upper left vertex.
+struct KeptQuad {
+    const float *tv, *v;
+};
+__device__ inline KeptQuad kept_quad(const RasterWS& ws, uint32_t wi, uint32_t ij) {
+    const float* p = ws.vbuf + (size_t)wi * kItemFloats;
+    const uint32_t lr = (ij >> 16) & 3u, q = (lr << 6) | (ij & 63u);
+    return {p + 2u * q, p + kItemTv + __umul24(q + lr, 3u)};
 }
 
-// Vertex block of quad (i, j) of pair vs when its work item was kept, else null.
-__device__ inline const float* kept_block(const RasterWS& ws, const BatchDims& d, uint32_t vs, int i, int j) {
-    const uint32_t wi = kept_index(ws, d, vs, i, j);
-    return wi == 0xffffffffu ? nullptr : ws.vbuf + (size_t)wi * (3 * kBinVerts);
+// Vertex window of quad ij of pair vs when its work item was kept, else null.
+__device__ inline const float* kept_block(const RasterWS& ws, const BatchDims& d, uint32_t vs, uint32_t ij) {
+    const uint32_t wi = kept_index(ws, d, vs, ij);
+    return wi == 0xffffffffu ? nullptr : kept_window(ws, wi);
 }
 
-// Validities of triangles T1, T2 of quad (i, j) of kept item wi (the counting
-// pass evaluated them exactly; only alive triangles' values are meaningful).
-__device__ inline float2 kept_validity(const RasterWS& ws, uint32_t wi, int i, int j) {
-    return ws.tvq[(size_t)wi * 256 + (uint32_t)((i % kBinQY) * kBinQX + (j % kBinQX))];
+// Corners a, b, c of slot 0 (v00 v01 v10) or 1 (v11 v10 v01) of a kept quad.
+__device__ inline void kept_corners(const float* v, int slot, float3 (&c)[3]) {
+    c[0] = load3(v + (slot ? 3 * (kBinQX + 2) : 0));
+    c[1] = load3(v + (slot ? 3 * (kBinQX + 1) : 3));
+    c[2] = load3(v + (slot ? 3 : 3 * (kBinQX + 1)));
 }
 
 // Vertices (i, sw - 1) and (i + 1, sw - 1) of pair vs, every item being kept:
 // from the window of the last quad of the row.
 __device__ inline void kept_seam(const RasterWS& ws, const BatchDims& d, uint32_t vs, int i, int sw, float3 (&l)[2]) {
-    const float* p = kept_quad(ws, kept_index<true>(ws, d, vs, i, sw - 2), i, sw - 2) + 3;
+    const uint32_t ij = ((uint32_t)i << 16) | (uint32_t)(sw - 2);
+    const float* p = kept_quad(ws, kept_index<true>(ws, d, vs, ij), ij).v + 3;
     l[0] = load3(p);
     l[1] = load3(p + 3 * (kBinQX + 1));
 }
@@ -578,7 +591,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
         int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;
         // a kept item also records its vertices and its quads' triangle validities for the raster
         {
-            float* vb = stored_geom ? ws.vbuf + (size_t)wi * (3 * kBinVerts) : nullptr;
+            float* vb = stored_geom ? kept_window(ws, wi) : nullptr;
 #pragma unroll 1
             for (int k = tid; k < kBinVerts; k += 256) {
                 const int rr = k / (kBinQX + 1), c = k % (kBinQX + 1);
@@ -595,7 +608,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
                 const int r = tid / kBinQX, c = tid % kBinQX;
                 more = quad_range_tv(g, i, j, V[r][c], V[r][c + 1], V[r + 1][c], V[r + 1][c + 1], vd.w, vd.h,
                                      d.tile_shift, tx0, tx1, ty0, ty1, stored_geom ? &tv : nullptr);
-                if (stored_geom) ws.tvq[(size_t)wi * 256 + tid] = tv;
+                if (stored_geom) {
+                    float* t = ws.vbuf + (size_t)wi * kItemFloats + 2 * tid;
+                    t[0] = tv.x; t[1] = tv.y;
+                }
             }
         }
         auto tile_of = [&](int tx, int ty) { return vd.tile_base + (uint32_t)(ty * vd.tiles_x + tx); };
@@ -765,7 +781,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
                     unpack_ij(w.quad, i, j);
                     float3 c[4];
                     if (d.kept_geom) {
-                        const float* p = kept_quad(ws, (uint32_t)b0 + (uint32_t)o * gridDim.x, i, j);
+                        const float* p = kept_quad(ws, (uint32_t)b0 + (uint32_t)o * gridDim.x, w.quad).v;
                         c[0] = load3(p); c[1] = load3(p + 3);
                         c[2] = load3(p + 3 * (kBinQX + 1)); c[3] = load3(p + 3 * (kBinQX + 1) + 3);
                     } else {
@@ -910,6 +926,26 @@ __device__ inline int lane_now() {
     return l;
 }
 
+// Colours of the corners of slot `slot` of source quad (i, j) (slot_vertex).
+template <class G>
+__device__ __forceinline__ void slot_colors(const G& g, int slot, int i, int j, float3 (&col)[3]) {
+    uint32_t idx[3];
+    if (slot < 2) {
+        const uint32_t p = (uint32_t)i * (uint32_t)g.sw + (uint32_t)j, down = (uint32_t)g.sw;
+        idx[0] = p + (slot ? down + 1u : 0u);
+        idx[1] = p + (slot ? down : 1u);
+        idx[2] = p + (slot ? 1u : down);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            int r, c;
+            slot_vertex(slot, k, i, j, g.sw, r, c);
+            idx[k] = (uint32_t)r * (uint32_t)g.sw + (uint32_t)c;
+        }
+    }
+    color3(g, idx, col);
+}
+
 // Winner's colour, depth and validity at pixel (x, y) for slot `slot` of
 // source quad (i, j): the state the fold holds after accepting that candidate.
 // FAST: vertex radii and the validity take only their fast float-float paths,
@@ -919,12 +955,9 @@ __device__ inline int lane_now() {
 template <bool FAST, class G>
 __device__ __forceinline__ bool resolve(const G& g, int i, int j, int slot, int x, int y, float3& c, float& dep,
                                float& shape, int out_w, int out_h, const float* vb) {
-    int r[3], cc[3];
     float3 v[3], col[3];
     bool und = false;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) slot_vertex(slot, k, i, j, g.sw, r[k], cc[k]);
-    color3(g, r, cc, col);   // issued first: its loads overlap the vertices'
+    slot_colors(g, slot, i, j, col);   // issued first: its loads overlap the vertices'
 #pragma unroll 1
     for (int k = 0; k < 3; ++k) {
         int rk, ck;
@@ -950,16 +983,13 @@ __device__ __forceinline__ bool resolve(const G& g, int i, int j, int slot, int 
     return true;
 }
 
-// The same from the corner vertices and validity the coverage pass cached
+// The same from the corner vertices and validity the counting pass kept
 // (identical float operations, without re-evaluating vertices or norms).
 template <class G>
 __device__ __forceinline__ void resolve_cached(const G& g, int i, int j, int slot, float3 a, float3 b, float3 cv, float tv,
                                       int x, int y, float3& c, float& dep, float& shape) {
-    int r[3], cc[3];
     float3 col[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) slot_vertex(slot, k, i, j, g.sw, r[k], cc[k]);
-    color3(g, r, cc, col);
+    slot_colors(g, slot, i, j, col);
     Tri T;
     tri_load(T, a, b, cv);
     T.tv = tv;
@@ -974,28 +1004,24 @@ __device__ __forceinline__ void resolve_cached(const G& g, int i, int j, int slo
 // score: scores are finite positive floats).
 constexpr uint32_t kDeferKey = 0xffffffffu;
 
-// Pushes candidate `id` of triangle T for pixel (x, y) of the tile at (tx0,
-// ty0): the exact coverage test, then the key updates.  r: recip(T.den), or 0
-// when T.den is outside quot_den's range.
-template <int TILE>
-__device__ __forceinline__ void raster_push(const Tri& T, float r, bool special, uint32_t id, int x, int y, int tx0,
-                                            int ty0, unsigned long long* key1, uint32_t* key2) {
-    float n1, n2, l1, l2, l3;
-    tri_num(T, x, y, n1, n2);
-    if (!(r != 0.f ? tri_cover_r(T, r, n1, n2, l1, l2, l3) : tri_cover(T, n1, n2, l1, l2, l3))) return;
-    const int p = (y - ty0) * TILE + (x - tx0);
+// Pushes candidate `id` of triangle T for the tile's pixel p with centre (fx,
+// fy): the exact coverage test, then the key updates.  r: recip(T.den).
+__device__ __forceinline__ void raster_push(const Tri& T, float r, bool special, uint32_t id, float fx, float fy, int p,
+                                            unsigned long long* key1, uint32_t* key2) {
+    // tri_num at the pixel
+    const float dx = fx - T.C0, dy = fy - T.C1;
+    const float n1 = (T.B1 - T.C1) * dx + (T.C0 - T.B0) * dy, n2 = (T.C1 - T.A1) * dx + (T.A0 - T.C0) * dy;
+    float l1, l2, l3;
+    if (!tri_cover_r(T, r, n1, n2, l1, l2, l3)) return;
     const float dd = tri_depth(T, l1, l2, l3);
-    if (special || !depth_regular(dd)) {
-        atomicMax(&key2[p], kDeferKey);
-        return;
-    }
     // the score only orders candidates outside the ambiguity band:
     // v_rcp_f32 (1 ulp) keeps its error within 5 * 2^-24 relative
     const float f = T.tv * __builtin_amdgcn_rcpf(dd * dd * dd);
-    const unsigned long long k = ((unsigned long long)f2u(f) << 32) | id;
+    const bool defer = special || !depth_regular(dd);
+    const unsigned long long k = defer ? 0ull : ((unsigned long long)f2u(f) << 32) | id;
     const unsigned long long old = atomicMax(&key1[p], k);
     // the candidate that is not (or no longer) the maximum goes to the runner-up slot
-    atomicMax(&key2[p], (uint32_t)((old < k ? old : k) >> 32));
+    atomicMax(&key2[p], defer ? kDeferKey : (uint32_t)((old < k ? old : k) >> 32));
 }
 
 // Ids of a phase's wide triangles, put off until its other triangles are done.
@@ -1011,13 +1037,6 @@ template <int TILE>
 __device__ __forceinline__ bool tile_box(Tri& T, int tx0, int ty0, int out_w, int out_h, int& xa, int& xb, int& ya,
                                          int& yb) {
     return tri_box(T, out_w, out_h, tx0, min(out_w, tx0 + TILE) - 1, ty0, min(out_h, ty0 + TILE) - 1, xa, xb, ya, yb);
-}
-
-// Whether pixel (x, y) may pass T's coverage test (r as in raster_push).
-__device__ __forceinline__ bool may_cover(const Tri& T, float r, int x, int y) {
-    float n1, n2;
-    tri_num(T, x, y, n1, n2);
-    return r != 0.f ? !tri_outside_r(r, n1, n2) : !tri_surely_outside(T, n1, n2);
 }
 
 // T's validity: the one the counting pass kept (> 0; KNOWN: it was evaluated
@@ -1051,27 +1070,37 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
     const bool prol = (a.z > 0.f) || (b.z > 0.f) || (c.z > 0.f);
     // a finite den has finite image coordinates
     bool special = !is_finite(a.z + b.z + c.z) || !is_finite(T.den) || (prol_false_possible && !prol) || undecided;
-    if (Q && !special && (xb - xa + 1) * (yb - ya + 1) > kWidePx) {
+    if (!cover_den(T.den)) {
+        // degenerate, gigantic or non-finite: whatever it may cover is deferred
+        for (int y = ya; y <= yb; ++y)
+            for (int x = xa; x <= xb; ++x) {
+                float n1, n2;
+                tri_num(T, x, y, n1, n2);
+                if (!tri_surely_outside(T, n1, n2)) atomicMax(&key2[(y - ty0) * TILE + (x - tx0)], kDeferKey);
+            }
+        return;
+    }
+    if (Q && !special && (int)__umul24(xb - xa + 1, yb - ya + 1) > kWidePx) {
         const uint32_t q = atomicAdd(&Q->n, 1u);
         if (q < Queue::cap) {
             Q->id[q] = id;
             return;
         }
     }
-    const float r = quot_den(T.den) ? recip(T.den) : 0.f;
+    const float r = recip(T.den);
     const float ex1 = T.B1 - T.C1, ey1 = T.C0 - T.B0, ex2 = T.C1 - T.A1, ey2 = T.A0 - T.C0;   // tri_num's
     T.tv = -1.f;   // not taken yet
-    // 8 x 8 pixels at a time (nearly every box is smaller), in two steps, so
-    // that lanes with few candidates do not wait through the exact test of
-    // lanes with large boxes: the rejection by approximate barycentrics marks
-    // the candidates (a bit each), then only those take the exact coverage test
-    // and the key updates.
-    for (int y0 = ya; y0 <= yb; y0 += 8)
+    // 8 x 4 pixels at a time (most boxes are smaller), in two steps, so that
+    // lanes with few candidates do not wait through the exact test of lanes
+    // with large boxes: the rejection by approximate barycentrics marks the
+    // candidates (a bit each), then only those take the exact coverage test and
+    // the key updates.
+    for (int y0 = ya; y0 <= yb; y0 += 4)
         for (int x0 = xa; x0 <= xb; x0 += 8) {
-            const int nx = min(xb - x0, 7), ny = min(yb - y0, 7);
-            const float fx0 = (float)x0 + 0.5f;
-            float fy = (float)y0 + 0.5f;
-            uint64_t mask = 0ull;
+            const int nx = min(xb - x0, 7), ny = min(yb - y0, 3);
+            const float fx0 = (float)x0 + 0.5f, fy0 = (float)y0 + 0.5f;
+            float fy = fy0;
+            uint32_t mask = 0u;
             for (int row = 0; row <= ny; ++row) {
                 const float dy = fy - T.C1, m1 = ey1 * dy, m2 = ey2 * dy;
                 float fx = fx0;
@@ -1081,15 +1110,16 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
                     if (!tri_outside_r(r, ex1 * dx + m1, ex2 * dx + m2)) bits |= bit;
                     fx += 1.f;
                 }
-                mask |= (uint64_t)bits << (row * 8);
+                mask |= bits << (row * 8);
                 fy += 1.f;
             }
             if (!mask) continue;
             if (T.tv < 0.f && !take_validity<KNOWN>(T, rescale, tv_known)) special = true;
+            const int p0 = (y0 - ty0) * TILE + (x0 - tx0);
             while (mask) {
-                const int bit = __builtin_ctzll(mask);
-                mask &= mask - 1ull;
-                raster_push<TILE>(T, r, special, id, x0 + (bit & 7), y0 + (bit >> 3), tx0, ty0, key1, key2);
+                const int bit = __builtin_ctz(mask), col = bit & 7, row = bit >> 3;
+                mask &= mask - 1u;
+                raster_push(T, r, special, id, fx0 + (float)col, fy0 + (float)row, p0 + row * TILE + col, key1, key2);
             }
         }
 }
@@ -1097,6 +1127,22 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
 __device__ __forceinline__ float lane_f(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
+
+// Bins of the sources of a phase, concatenated: source k's entries e lie in
+// [end[k - 1], end[k]) and at lists[e + add[k]] (modulo 2^32).  Uniform: in SGPRs.
+struct Phase {
+    uint32_t end0, end1, end2, n;
+    uint32_t add0, d1, d2, d3;   // add[0], and each later source's step (selects between the sums
+                                 // themselves become loads from scratch)
+    // Source of entry e < n and its quad code.
+    __device__ int find(const RasterWS& ws, uint32_t e, uint32_t& code) const {
+        const bool a = e >= end0, b = e >= end1, c = e >= end2;
+        const uint32_t at = add0 + (a ? d1 : 0u) + (b ? d2 : 0u) + (c ? d3 : 0u);
+        code = ws.lists[e + at];
+        return (int)a + (int)b + (int)c;
+    }
+};
+static_assert(kRasterGroup == 4 && kRasterGroupMulti == 4, "a phase of four sources");
 
 // The wave's share of a phase's queued triangles: each lane fetches and sets
 // up one (a single chain of loads for all of them), then the wave takes them
@@ -1107,8 +1153,7 @@ __device__ __forceinline__ float lane_f(float v, int lane) {
 // Measured: two 3840x2160 views of 11 perspective sources, raster 4.03 -> 3.40
 // ms; 8 views of 1920x1080 of four panoramas 1.80 -> 1.22 ms.
 template <int TILE, int NT, bool KEPT, class G, class Queue>
-__device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, const uint32_t* pref, int gs,
-                                            uint32_t nwide, const Queue& Q, int wave, int tx0, int ty0, int out_w,
+__device__ __forceinline__ void raster_wide(const G* gv, const Phase& ph, uint32_t nwide, const Queue& Q, int wave, int tx0, int ty0, int out_w,
                                             int out_h, unsigned long long (*key1)[NT], uint32_t (*key2)[NT],
                                             const RasterWS& ws, const BatchDims& d, uint32_t vs0) {
     constexpr uint32_t NW = NT / 64;
@@ -1120,24 +1165,21 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
         uint32_t id = 0u;
         if (q < nwide) {
             id = Q.id[q];
-            const uint32_t e = id >> 2;
-            while (k + 1 < gs && e >= pref[k + 1]) ++k;
+            uint32_t code;
+            k = ph.find(ws, id >> 2, code);
             int i, j;
-            unpack_ij(ws.lists[(size_t)boff[k] + (e - pref[k])], i, j);
+            unpack_ij(code, i, j);
             const G& g = gv[k];
-            const uint32_t wi = kept_index<KEPT>(ws, d, vs0 + (uint32_t)k, i, j);
-            // the corners of slot 0 (v00 v01 v10) or 1 (v11 v10 v01); one evaluated
-            // here was decided by the fast path when the triangle was queued
+            const uint32_t wi = kept_index<KEPT>(ws, d, vs0 + (uint32_t)k, code);
+            // one evaluated here was decided by the fast path when the triangle was queued
             const int slot = (int)(id & 3u);
             bool und = false;
             float2 tvk = make_float2(0.f, 0.f);
             float3 c3[3];
             if (KEPT || wi != 0xffffffffu) {
-                const float* p = kept_quad(ws, wi, i, j);
-                c3[0] = load3(p + (slot ? 3 * (kBinQX + 2) : 0));
-                c3[1] = load3(p + (slot ? 3 * (kBinQX + 1) : 3));
-                c3[2] = load3(p + (slot ? 3 : 3 * (kBinQX + 1)));
-                tvk = kept_validity(ws, wi, i, j);
+                const KeptQuad kq = kept_quad(ws, wi, code);
+                kept_corners(kq.v, slot, c3);
+                tvk = make_float2(kq.tv[0], kq.tv[1]);
             } else {
                 eval_corners<3>(g, i, j, slot ? 3u : 4u, slot ? 5u : 2u, c3, &und);
             }
@@ -1145,7 +1187,7 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
             tri_load(T, a, b, c);
             tile_box<TILE>(T, tx0, ty0, out_w, out_h, xa, xb, ya, yb);
             if (!take_validity<KEPT>(T, g.rescale, slot ? tvk.y : tvk.x)) sp = 0x100;
-            if (quot_den(T.den)) tr = recip(T.den);
+            tr = recip(T.den);
         }
         const int m = min(64, (int)((nwide - q0 + NW - 1u) / NW));
         for (int l = 0; l < m; ++l) {
@@ -1165,8 +1207,11 @@ __device__ __forceinline__ void raster_wide(const G* gv, const uint32_t* boff, c
                 // row i / bw: i + 1/2 is at least 1 / (2 bw) of a row away from the next one
                 const int row = (int)(((float)i + 0.5f) * inv);
                 const int x = wx + (i - row * bw), y = wy + row;
-                if (may_cover(W, r, x, y))
-                    raster_push<TILE>(W, r, sk >= 0x100, wid, x, y, tx0, ty0, key1[sk & 0xff], key2[sk & 0xff]);
+                float n1, n2;
+                tri_num(W, x, y, n1, n2);
+                if (!tri_outside_r(r, n1, n2))
+                    raster_push(W, r, sk >= 0x100, wid, (float)x + 0.5f, (float)y + 0.5f,
+                                (y - ty0) * TILE + (x - tx0), key1[sk & 0xff], key2[sk & 0xff]);
             }
         }
     }
@@ -1195,17 +1240,18 @@ __device__ __forceinline__ void raster_quad(const G& g, const G& gt, uint32_t ij
                                             Queue* Q, const RasterWS& ws, const BatchDims& d, uint32_t vs) {
     int i, j;
     unpack_ij(ij, i, j);
-    const uint32_t wi = kept_index<KEPT>(ws, d, vs, i, j);
+    const uint32_t wi = kept_index<KEPT>(ws, d, vs, ij);
     // vertices evaluated here take the fast radius path; an undecided one
     // defers the pixels of the quad's triangles (kept vertices are exact)
     bool und = false;
     float2 tvk = make_float2(0.f, 0.f);
     float3 v00, v01, v10, v11;
     if (KEPT || wi != 0xffffffffu) {
-        const float* p = kept_quad(ws, wi, i, j);
+        const KeptQuad kq = kept_quad(ws, wi, ij);
+        const float* p = kq.v;
         v00 = load3(p); v01 = load3(p + 3);
         v10 = load3(p + 3 * (kBinQX + 1)); v11 = load3(p + 3 * (kBinQX + 1) + 3);
-        tvk = kept_validity(ws, wi, i, j);
+        tvk = make_float2(kq.tv[0], kq.tv[1]);
     } else {
         float3 v[4];
         eval_corners<4>(g, i, j, 0xcu, 0xau, v, &und);
@@ -1293,8 +1339,6 @@ struct RasterLds {
     static constexpr int GRP = MULTI ? kRasterGroupMulti : kRasterGroup;   // sources per phase
     unsigned long long key1[GRP][NT];
     uint32_t key2[GRP][NT];
-    uint32_t pref[GRP + 1];
-    uint32_t boff[GRP];   // list offsets of the phase's bins
     int s_deferred;       // any pixel of the tile deferred
     int s_hole;           // any pixel of the tile a hole (quality not > 0)
     // one phase: a smaller cache keeps a 16 x 16 block within 20 KB of LDS (8 blocks per CU)
@@ -1306,10 +1350,14 @@ struct RasterLds {
 // One tile of k_raster.  Bound by the issue of VALU instructions (0.62 T/s of wave
 // instructions; 1024 SIMDs issue 0.61 T/s at 2.4 GHz).  Raster ms with the box and the narrowing one
 // after the other, the candidates marked by exact numerators and every
-// barycentric divided out, vertex code in one body -> now: 16 views of mixed
-// sizes 3.13 -> 2.57, one 1920x1080 view 0.246 -> 0.194 (four 4096x2048
-// panoramas); 8192x4096 panorama of eleven 11.0 -> 7.9; two 3840x2160 views of
-// 11 perspective sources 3.42 -> 2.87.  KEPT: every surviving work item keeps its vertex
+// barycentric divided out, vertex code in one body, 64-bit index arithmetic and
+// branches in the candidate and blend loops -> now: 16 views of mixed sizes
+// 3.13 -> 2.38, one 1920x1080 view 0.246 -> 0.177 (four 4096x2048 panoramas);
+// 8192x4096 panorama of eleven 11.0 -> 7.3; two 3840x2160 views of 11
+// perspective sources 3.42 -> 2.66.  Of 2.57 ms (16 views, builds that skip a
+// part): resolve and blend 0.75, exact tests and keys 0.56, vertex fetch and
+// denominators 0.41, candidate scan 0.34, wide triangles 0.13, boxes 0.07, the
+// rest of a tile 0.37.  KEPT: every surviving work item keeps its vertex
 // window and validities (nearly always), so this code evaluates no vertex and
 // no validity of slots 0 and 1: a third of the instructions of the general
 // form, whose registers would otherwise spill around them.
@@ -1321,8 +1369,6 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
     constexpr int NT = Lds::NT, GRP = Lds::GRP;
     auto& key1 = L.key1;
     auto& key2 = L.key2;
-    auto& pref = L.pref;
-    auto& boff = L.boff;
     auto& cache = L.cache;
     Queue& wide = L.wide;
     int& s_deferred = L.s_deferred;
@@ -1351,42 +1397,34 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
         if (tid == 0) {
             if (s0 == 0) { s_deferred = 0; s_hole = 0; }
             wide.n = 0u;
-            // the phase's counts and offsets loaded together, then summed
-            uint32_t cnt[GRP], off[GRP];
-#pragma unroll
-            for (int k = 0; k < GRP; ++k) {
-                const size_t b = bin_index(d, T, (uint32_t)(s0 + (k < gs ? k : 0)));
-                cnt[k] = ws.counts[b];
-                off[k] = ws.offsets[b];
-            }
-            uint32_t acc = 0;
-#pragma unroll
-            for (int k = 0; k < GRP; ++k)
-                if (k < gs) {
-                    pref[k] = acc;
-                    boff[k] = off[k];
-                    acc += cnt[k];
-                }
-            pref[gs] = acc;
         }
+        uint32_t end[GRP], add[GRP], acc = 0u;
+#pragma unroll
+        for (int k = 0; k < GRP; ++k) {
+            const size_t b = bin_index(d, T, (uint32_t)(s0 + (k < gs ? k : 0)));
+            const uint32_t cnt = ws.counts[b], off = ws.offsets[b];
+            add[k] = off - acc;
+            acc += k < gs ? cnt : 0u;
+            end[k] = acc;
+        }
+        const Phase ph = {end[0], end[1], end[2], acc, add[0], add[1] - add[0], add[2] - add[1], add[3] - add[2]};
         __syncthreads();
-        const uint32_t N = __builtin_amdgcn_readfirstlane(pref[gs]);   // uniform: kept in an SGPR
+        const uint32_t N = ph.n;
         const bool cached = N <= (uint32_t)cache.cap;
         // a wave-uniform trip count; the entry index is re-derived each trip
         const uint32_t trips = (N + (uint32_t)NT - 1u) / (uint32_t)NT;
         for (uint32_t it = 0; it < trips; ++it) {
             const uint32_t e = it * (uint32_t)NT + (uint32_t)(wave_base + lane_now());
             if (e >= N) continue;
-            int k = 0;
-            while (k + 1 < gs && e >= pref[k + 1]) ++k;
-            const uint32_t ij = ws.lists[(size_t)boff[k] + (e - pref[k])];
+            uint32_t ij;
+            const int k = ph.find(ws, e, ij);
             raster_quad<TILE, KEPT>(gv[s0 + k], gv[0], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k], cached ? &cache : nullptr,
                               &wide, ws, d, (uint32_t)(v * d.nsrc + s0 + k));
         }
         __syncthreads();
         const uint32_t nwide = __builtin_amdgcn_readfirstlane(min(wide.n, Queue::cap));
         if (nwide) {   // the same in every wave
-            raster_wide<TILE, NT, KEPT>(gv + s0, boff, pref, gs, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1,
+            raster_wide<TILE, NT, KEPT>(gv + s0, ph, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1,
                                   key2, ws, d, (uint32_t)(v * d.nsrc + s0));
             __syncthreads();
         }
@@ -1412,22 +1450,21 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
                     const int slot = (int)(id & 3u);
                     const G& g = gv[s];
                     const uint32_t vs = (uint32_t)(v * d.nsrc + s);
-                    const uint32_t ij = cached ? cache.ij[e] : ws.lists[(size_t)boff[k] + (e - pref[k])];
+                    uint32_t ij;
+                    if (cached) ij = cache.ij[e];
+                    else ph.find(ws, e, ij);
                     int i, j;
                     unpack_ij(ij, i, j);
-                    const uint32_t wk = cached ? cache.wi[e] : kept_index<KEPT>(ws, d, vs, i, j);
+                    const uint32_t wk = cached ? cache.wi[e] : kept_index<KEPT>(ws, d, vs, ij);
                     bool ok = true;
                     if (slot < 2 && (KEPT || wk != 0xffffffffu)) {
-                        // T1: v00 v01 v10; T2: v11 v10 v01 (corner offsets of slot_vertex);
                         // the validity the counting pass kept (the coverage pass used it)
-                        const float* p = kept_quad(ws, wk, i, j);
-                        const float3 a = load3(p + (slot ? 3 * (kBinQX + 2) : 0));
-                        const float3 b = load3(p + (slot ? 3 * (kBinQX + 1) : 3));
-                        const float3 cc = load3(p + (slot ? 3 : 3 * (kBinQX + 1)));
-                        const float2 tvk = kept_validity(ws, wk, i, j);
-                        resolve_cached(g, i, j, slot, a, b, cc, slot ? tvk.y : tvk.x, px, py, c, dep, shape);
+                        const KeptQuad kq = kept_quad(ws, wk, ij);
+                        float3 t[3];
+                        kept_corners(kq.v, slot, t);
+                        resolve_cached(g, i, j, slot, t[0], t[1], t[2], kq.tv[slot], px, py, c, dep, shape);
                     } else if (KEPT) {   // slot 2: l0 v00 l1, slot 3: v10 l1 v00
-                        const float* p = kept_quad(ws, wk, i, j);
+                        const float* p = kept_quad(ws, wk, ij).v;
                         const float3 v00 = load3(p), v10 = load3(p + 3 * (kBinQX + 1));
                         float3 l[2];
                         kept_seam(ws, d, vs, i, g.sw, l);
@@ -1437,7 +1474,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
                         ok = tri_validity_fast(T, g.rescale, T.tv);
                         resolve_cached(g, i, j, slot, a, b, cc, T.tv, px, py, c, dep, shape);
                     } else {
-                        ok = resolve<true>(g, i, j, slot, px, py, c, dep, shape, vd.w, vd.h, kept_block(ws, d, vs, i, j));
+                        ok = resolve<true>(g, i, j, slot, px, py, c, dep, shape, vd.w, vd.h, kept_block(ws, d, vs, ij));
                     }
                     if (!ok) { deferred = true; break; }
                 }
@@ -1577,7 +1614,7 @@ __device__ void replay_source(const G& g, uint32_t* L, uint32_t n, int tx0, int 
             const uint32_t q = L[e];
             int i, j;
             unpack_ij(q, i, j);
-            const float* vb = kept_block(ws, d, vs, i, j);
+            const float* vb = kept_block(ws, d, vs, q);
             const int r0 = i - i % kBinQY, c0 = j - j % kBinQX;
             auto vtx = [&](int ii, int jj) { return kept_or_eval(vb, r0, c0, ii, jj); };
             quad_tris(g, i, j, vtx, out_w, out_h, [&](int k, Tri& Tr, bool prol) {
@@ -1679,7 +1716,7 @@ __device__ void replay_source(const G& g, uint32_t* L, uint32_t n, int tx0, int 
             int i, j;
             unpack_ij(q, i, j);
             Quad Q;
-            const float* vb = kept_block(ws, d, vs, i, j);
+            const float* vb = kept_block(ws, d, vs, q);
             const int r0 = i - i % kBinQY, c0 = j - j % kBinQX;
             auto vtx = [&](int ii, int jj) { return kept_or_eval(vb, r0, c0, ii, jj); };
             quad_build(Q, g, i, j, vtx, out_w, out_h);

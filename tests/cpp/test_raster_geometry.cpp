@@ -88,7 +88,7 @@ int main() {
         int xa = 0, xb = W - 1, ya = 0, yb = H - 1;
         const bool box = tri_near_box(A0, A1, B0, B1, C0, C1, den, 0, W - 1, 0, H - 1, xa, xb, ya, yb);
         boxed += box;
-        const bool fast = quot_den(den);
+        const bool fast = cover_den(den);
         const float r = fast ? recip(den) : 0.f;
         for (int y = ymin; y <= ymax; ++y)
             for (int x = xmin; x <= xmax; ++x) {
@@ -107,7 +107,7 @@ int main() {
                 const float q1 = quot(n1, den, r), q2 = quot(n2, den, r), q3 = 1.f - q1 - q2;
                 const bool qin = q1 >= -1e-6f && q2 >= -1e-6f && q3 >= -1e-6f;
                 if (qin != in) ++wrong;
-                if (in && quot_num(n1) && quot_num(n2) && (f2u(q1) != f2u(l1) || f2u(q2) != f2u(l2))) ++wrong;
+                if (in && quot_den(den) && quot_num(n1) && quot_num(n2) && (f2u(q1) != f2u(l1) || f2u(q2) != f2u(l2))) ++wrong;
             }
     }
     std::printf("quotients %ld wrong; boxes %ld, covered %ld, outside %ld; rejected %ld, missed %ld; coverage %ld wrong\n",
