@@ -184,7 +184,10 @@ void Server::reset(const rvs_request* reqs, int n) {
     m_errmsg.clear();
     m_pending.clear();
     m_stats.assign(n, rvs_request_stats{});
-    m_out.assign(m_opt.keep_outputs ? n : 0, std::vector<uint8_t>());
+    // the kept outputs' buffers serve run after run: fresh ones would be paged
+    // in again for every request
+    m_out.resize(m_opt.keep_outputs ? n : 0);
+    for (std::vector<uint8_t>& o : m_out) o.clear();
     for (int k = 0; k < n; ++k) {
         m_stats[k].rc = 1;   // not done
         if (reqs[k].scene < 0 || reqs[k].scene >= (int)m_scenes.size())

@@ -106,9 +106,17 @@ class Server:
         n = _lib().rvs_server_output(self.h, int(k), None, 0)
         if n < 0:
             raise RuntimeError("no output kept for request %d" % k)
-        buf = (C.c_uint8 * n)()
-        _lib().rvs_server_output(self.h, int(k), buf, n)
-        return bytes(buf)
+        out = _new_bytes(None, n)   # not yet seen by anyone else, so it may be written
+        _lib().rvs_server_output(self.h, int(k), _bytes_at(out), n)
+        return out
+
+
+# An uninitialised bytes object and its buffer: one copy of an output instead
+# of a zeroed array, a copy into it and a copy out of it.
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.argtypes, _new_bytes.restype = [C.c_char_p, C.c_ssize_t], C.py_object
+_bytes_at = C.pythonapi.PyBytes_AsString
+_bytes_at.argtypes, _bytes_at.restype = [C.py_object], C.c_void_p
 
 
 def summarize(stats, wall_s=None):
