@@ -96,11 +96,14 @@ __device__ inline uint32_t load_plane(const void* p, int u8, size_t idx) {
 
 // Source pixel (i = row, j = column) unprojected into the source camera frame
 // (decode depth, then EquirectangularUnprojector / PerspectiveUnprojector).
-__device__ inline float3 unproject_src(const PairGeom& g, int i, int j) {
+__device__ inline float src_depth(const PairGeom& g, int i, int j) {
     const size_t idx = (size_t)i * g.sw + j;
-    const float d = g.depth_f32 ? ((const float*)g.depth)[idx]
-                                : decode_depth_raw(load_plane(g.depth, g.depth_u8, idx), g.dscale, g.znear,
-                                                   g.zfar, g.has_invalid);
+    return g.depth_f32 ? ((const float*)g.depth)[idx]
+                       : decode_depth_raw(load_plane(g.depth, g.depth_u8, idx), g.dscale, g.znear, g.zfar,
+                                          g.has_invalid);
+}
+
+__device__ inline float3 unproject_depth(const PairGeom& g, int i, int j, float d) {
     float x, y, z;
     if (g.src_erp) {
         const float cp = g.tab[j], sp = g.tab[g.sw + j];
@@ -122,6 +125,10 @@ __device__ inline float3 unproject_src(const PairGeom& g, int i, int j) {
         }
     }
     return make_float3(x, y, z);
+}
+
+__device__ inline float3 unproject_src(const PairGeom& g, int i, int j) {
+    return unproject_depth(g, i, j, src_depth(g, i, j));
 }
 
 // Source-frame point -> target u', v' (after the uv rescale) and target depth.

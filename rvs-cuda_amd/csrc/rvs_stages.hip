@@ -7,45 +7,142 @@ namespace rvs_k {
 
 using namespace rvs_dev;
 
-// read_color_YUV -> resizeImage + mergeFrame (image_loading.cpp:74-145).
-__global__ void k_decode_color(const void* y, const void* u, const void* v, int u8, int w, int h, float cs,
-                               float* __restrict__ out) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int r = blockIdx.y;
-    if (x >= w || r >= h) return;
-    PairGeom g;
-    g.sw = w; g.sh = h; g.py = y; g.pu = u; g.pv = v; g.color_u8 = u8; g.cscale = cs; g.col = nullptr;
-    g.colq = nullptr;
-    const float3 c = color(g, r, x);
-    const size_t o = (size_t)r * w + x;
-    out[3 * o] = c.x; out[3 * o + 1] = c.y; out[3 * o + 2] = c.z;
-}
+// Writers of four horizontally adjacent decoded pixels (Y, U, V before the
+// colour scale): the float colour map, the resident plane of 16-bit integers
+// (exact for even sizes and codes below 2^14, whose upsampled chroma is a
+// multiple of 1/4), or the resident plane of floats.
+struct ColorOut {
+    float* p;
+    float cs;
+    __device__ void put(size_t o, float y, float u, float v) const {
+        p[3 * o] = y * cs; p[3 * o + 1] = u * cs; p[3 * o + 2] = v * cs;
+    }
+    __device__ void put4(size_t o, const float (&y)[4], const float (&u)[4], const float (&v)[4]) const {
+        float t[12];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { t[3 * k] = y[k] * cs; t[3 * k + 1] = u[k] * cs; t[3 * k + 2] = v[k] * cs; }
+        __builtin_memcpy(p + 3 * o, t, sizeof t);
+    }
+};
+struct PackedOut {
+    ushort4* p;
+    __device__ void put(size_t o, float y, float u, float v) const {
+        p[o] = make_ushort4((unsigned short)y, (unsigned short)(u * 4.f), (unsigned short)(v * 4.f), 0);
+    }
+    __device__ void put4(size_t o, const float (&y)[4], const float (&u)[4], const float (&v)[4]) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) put(o + k, y[k], u[k], v[k]);
+    }
+};
+struct FloatOut {
+    float4* p;
+    __device__ void put(size_t o, float y, float u, float v) const { p[o] = make_float4(y, u, v, 0.f); }
+    __device__ void put4(size_t o, const float (&y)[4], const float (&u)[4], const float (&v)[4]) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) put(o + k, y[k], u[k], v[k]);
+    }
+};
 
-// Resident decoded colour plane of a source (color_raw per pixel): floats, or
-// (packed) Y, 4 U, 4 V as 16-bit integers -- exact for even sizes and codes
-// below 2^14, whose upsampled chroma is a multiple of 1/4.
-__global__ void k_prep_color(const void* y, const void* u, const void* v, int u8, int w, int h, int packed,
-                             void* __restrict__ out) {
+// read_color_YUV -> resizeImage + mergeFrame (image_loading.cpp:74-145), any
+// size: a thread per pixel.
+template <class Out>
+__global__ void k_color(const void* y, const void* u, const void* v, int u8, int w, int h, Out out) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int r = blockIdx.y;
     if (x >= w || r >= h) return;
     PairGeom g;
     g.sw = w; g.sh = h; g.py = y; g.pu = u; g.pv = v; g.color_u8 = u8; g.col = nullptr; g.colq = nullptr;
     const float3 c = color_raw(g, r, x);
-    const size_t o = (size_t)r * w + x;
-    if (packed)
-        ((ushort4*)out)[o] = make_ushort4((unsigned short)c.x, (unsigned short)(c.y * 4.f),
-                                          (unsigned short)(c.z * 4.f), 0);
-    else
-        ((float4*)out)[o] = make_float4(c.x, c.y, c.z, 0.f);
+    out.put((size_t)r * w + x, c.x, c.y, c.z);
+}
+
+// The same for even sizes: a thread takes four pixels of two rows, whose chroma
+// needs three samples of two rows of each plane (color_raw's even form: the
+// sums and halves are exact, so the order does not matter).  Bound by HBM: 3 B
+// read and 8 (packed) or 12 B written per pixel.  A thread per pixel took up to
+// nine 1- or 2-byte loads each: 4096x2048 10-bit to the packed plane 61 -> 29 us,
+// 2048x2048 to the float map 25.7 -> 17.1 us.
+template <typename T, class Out>
+__global__ void __launch_bounds__(256) k_color_even(const T* __restrict__ Y, const T* __restrict__ U,
+                                                    const T* __restrict__ V, int w, int h, Out out) {
+    const int x = 4 * (int)(blockIdx.x * 64 + (threadIdx.x & 63));
+    const int r = 2 * (int)(blockIdx.y * 4 + (threadIdx.x >> 6));
+    if (x >= w || r >= h) return;
+    const int cw = w / 2, ch = h / 2, cx = x / 2, cy = r / 2;
+    const int x1 = min(cx + 1, cw - 1), x2 = min(cx + 2, cw - 1);
+    const size_t r0 = (size_t)cy * cw, r1 = (size_t)min(cy + 1, ch - 1) * cw;
+    // chroma of the upper row (even: its own samples) and the lower one (the
+    // mean with the next), at columns x .. x + 3
+    float c[2][2][4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const T* P = p ? V : U;
+        const float a0 = (float)P[r0 + cx], a1 = (float)P[r0 + x1], a2 = (float)P[r0 + x2];
+        const float b0 = (float)P[r1 + cx], b1 = (float)P[r1 + x1], b2 = (float)P[r1 + x2];
+        const float up[4] = {a0, (a0 + a1) * 0.5f, a1, (a1 + a2) * 0.5f};
+        const float lo[4] = {b0, (b0 + b1) * 0.5f, b1, (b1 + b2) * 0.5f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            c[p][0][k] = up[k];
+            c[p][1][k] = (up[k] + lo[k]) * 0.5f;
+        }
+    }
+#pragma unroll
+    for (int row = 0; row < 2; ++row) {
+        const size_t o = (size_t)(r + row) * w + x;
+        if (x + 4 <= w) {
+            T q[4];
+            __builtin_memcpy(q, Y + o, sizeof q);
+            const float l[4] = {(float)q[0], (float)q[1], (float)q[2], (float)q[3]};
+            out.put4(o, l, c[0][row], c[1][row]);
+        } else {   // the last two columns
+            out.put(o, (float)Y[o], c[0][row][0], c[1][row][0]);
+            out.put(o + 1, (float)Y[o + 1], c[0][row][1], c[1][row][1]);
+        }
+    }
+}
+
+template <class Out>
+hipError_t launch_color(const void* y, const void* u, const void* v, int u8, int w, int h, Out out, hipStream_t s) {
+    if (((w | h) & 1) == 0) {
+        const dim3 grid((w + 255) / 256, (h + 7) / 8);
+        if (u8)
+            hipLaunchKernelGGL((k_color_even<uint8_t, Out>), grid, dim3(256), 0, s, (const uint8_t*)y,
+                               (const uint8_t*)u, (const uint8_t*)v, w, h, out);
+        else
+            hipLaunchKernelGGL((k_color_even<uint16_t, Out>), grid, dim3(256), 0, s, (const uint16_t*)y,
+                               (const uint16_t*)u, (const uint16_t*)v, w, h, out);
+    } else {
+        hipLaunchKernelGGL(k_color<Out>, dim3((w + 255) / 256, h), dim3(256), 0, s, y, u, v, u8, w, h, out);
+    }
+    return hipGetLastError();
 }
 
 // read_depth_YUV -> formatDepth (image_loading.cpp:147-213).
 __global__ void k_decode_depth(const void* raw, int u8, size_t n, float scale, float znear, float zfar,
                                int has_invalid, float* __restrict__ out) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t i = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n) return;
-    out[i] = decode_depth_raw(load_plane(raw, u8, i), scale, znear, zfar, has_invalid);
+    if (i + 4 <= n) {
+        uint32_t q[4];
+        if (u8) {
+            uint8_t t[4];
+            __builtin_memcpy(t, (const uint8_t*)raw + i, sizeof t);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = t[k];
+        } else {
+            uint16_t t[4];
+            __builtin_memcpy(t, (const uint16_t*)raw + i, sizeof t);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = t[k];
+        }
+        float d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = decode_depth_raw(q[k], scale, znear, zfar, has_invalid);
+        __builtin_memcpy(out + i, d, sizeof d);
+        return;
+    }
+    for (size_t k = i; k < n; ++k) out[k] = decode_depth_raw(load_plane(raw, u8, k), scale, znear, zfar, has_invalid);
 }
 
 // SynthesizedView::computeBasicMode stage (a) (SynthesizedView.cpp:315-331).
@@ -161,19 +258,18 @@ hipError_t launch_resize_color(const float* src, int sw, int sh, float* dst, int
 
 hipError_t launch_decode_color(const void* y, const void* u, const void* v, int u8, int w, int h, float cs,
                                float* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_decode_color, dim3((w + 255) / 256, h), dim3(256), 0, s, y, u, v, u8, w, h, cs, out);
-    return hipGetLastError();
+    return launch_color(y, u, v, u8, w, h, ColorOut{out, cs}, s);
 }
 
 hipError_t launch_prep_color(const void* y, const void* u, const void* v, int u8, int w, int h, int packed,
                              void* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_prep_color, dim3((w + 255) / 256, h), dim3(256), 0, s, y, u, v, u8, w, h, packed, out);
-    return hipGetLastError();
+    if (packed) return launch_color(y, u, v, u8, w, h, PackedOut{(ushort4*)out}, s);
+    return launch_color(y, u, v, u8, w, h, FloatOut{(float4*)out}, s);
 }
 
 hipError_t launch_decode_depth(const void* raw, int u8, size_t n, float scale, float znear, float zfar,
                                int has_invalid, float* out, hipStream_t s) {
-    hipLaunchKernelGGL(k_decode_depth, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, raw, u8, n, scale, znear,
+    hipLaunchKernelGGL(k_decode_depth, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, raw, u8, n, scale, znear,
                        zfar, has_invalid, out);
     return hipGetLastError();
 }

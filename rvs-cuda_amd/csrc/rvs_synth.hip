@@ -227,35 +227,76 @@ __device__ inline void unpack_ij(uint32_t ij, int& i, int& j) {
 
 // ------------------------------------------------------------ culling
 
+// Minimum (MIN) or maximum over the wave, in its last lane: moves between
+// lanes as DPP operands instead of through LDS.
+template <bool MIN, int CTRL, int ROWS>
+__device__ inline float dpp_step(float v) {
+    const int m = __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xf, false);
+    return MIN ? min3f(v, v, __int_as_float(m)) : max3f(v, v, __int_as_float(m));
+}
+template <bool MIN>
+__device__ inline float wave_last(float v) {
+    v = dpp_step<MIN, 0x111, 0xf>(v);   // row_shr:1
+    v = dpp_step<MIN, 0x112, 0xf>(v);   // row_shr:2
+    v = dpp_step<MIN, 0x114, 0xf>(v);   // row_shr:4
+    v = dpp_step<MIN, 0x118, 0xf>(v);   // row_shr:8
+    v = dpp_step<MIN, 0x142, 0xa>(v);   // row_bcast:15 into rows 1, 3
+    return dpp_step<MIN, 0x143, 0xc>(v);   // row_bcast:31 into rows 2, 3
+}
+
 // Culling table of one source: per binning block (kBinQY x kBinQX quads), the
 // bounding box (source camera frame) of the finite unprojected points of its
 // vertex window (kBinQY+1 rows x kBinQX+1 columns) as min x, y, z, max x, y, z;
-// no finite point -> min +inf, max -inf.  One wave per block.
+// no finite point -> min +inf, max -inf.  One wave per block; bound by VALU
+// issue: 4096x2048 equirectangular 36 -> 30 us with the points in
+// pairs, the columns' tables loaded once and DPP reductions.
 __global__ void __launch_bounds__(256) k_src_bounds(PairGeom g, int bins_x, int bins_y, float* out) {
     const int lane = threadIdx.x & 63;
-    const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int item = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (item >= bins_x * bins_y) return;   // whole wave
     const int i0 = (item / bins_x) * kBinQY, j0 = (item % bins_x) * kBinQX;
-    float v[6] = {__builtin_inff(), __builtin_inff(), __builtin_inff(),
-                  -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-    for (int k = lane; k < (kBinQY + 1) * (kBinQX + 1); k += 64) {
-        const int i = i0 + k / (kBinQX + 1), j = j0 + k % (kBinQX + 1);
-        if (i >= g.sh || j >= g.sw) continue;
-        const float3 p = unproject_src(g, i, j);
-        if (!finite3(p)) continue;
-        v[0] = fminf(v[0], p.x); v[1] = fminf(v[1], p.y); v[2] = fminf(v[2], p.z);
-        v[3] = fmaxf(v[3], p.x); v[4] = fmaxf(v[4], p.y); v[5] = fmaxf(v[5], p.z);
+    const float inf = __builtin_inff();
+    float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+    // points in pairs; the minima pass over NaNs, and a point with any
+    // non-finite coordinate becomes NaNs
+    auto add = [&](float3 p, float3 q) {
+        const float n = __builtin_nanf("");
+        const bool a = is_finite(p.x + p.y + p.z), b = is_finite(q.x + q.y + q.z);
+        const float ps[3] = {a ? p.x : n, a ? p.y : n, a ? p.z : n}, qs[3] = {b ? q.x : n, b ? q.y : n, b ? q.z : n};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            lo[c] = min3f(lo[c], ps[c], qs[c]);
+            hi[c] = max3f(hi[c], ps[c], qs[c]);
+        }
+    };
+    const float none = __builtin_nanf("");
+    const float3 no_point = make_float3(none, none, none);
+    // a lane per column, the rows' depths loaded together; then the last column
+    const int j = j0 + lane;
+    float3 p[kBinQY + 2];
+#pragma unroll
+    for (int r = 0; r < kBinQY + 2; ++r) p[r] = no_point;
+    if (j < g.sw) {
+        float d[kBinQY + 1];
+#pragma unroll
+        for (int r = 0; r <= kBinQY; ++r) d[r] = src_depth(g, min(i0 + r, g.sh - 1), j);
+#pragma unroll
+        for (int r = 0; r <= kBinQY; ++r) p[r] = unproject_depth(g, min(i0 + r, g.sh - 1), j, d[r]);   // a row twice: the same box
     }
+    if (lane <= kBinQY && i0 + lane < g.sh && j0 + kBinQX < g.sw)
+        p[kBinQY + 1] = unproject_src(g, i0 + lane, j0 + kBinQX);
+    static_assert(kBinQY == 4, "three pairs");
+    add(p[0], p[1]); add(p[2], p[3]); add(p[4], p[5]);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) v[c] = fminf(v[c], __shfl_xor(v[c], off));
-#pragma unroll
-        for (int c = 3; c < 6; ++c) v[c] = fmaxf(v[c], __shfl_xor(v[c], off));
+    for (int c = 0; c < 3; ++c) {
+        lo[c] = wave_last<true>(lo[c]);
+        hi[c] = wave_last<false>(hi[c]);
     }
-    if (lane == 0)
-#pragma unroll
-        for (int c = 0; c < 6; ++c) out[(size_t)item * 6 + c] = v[c];
+    if (lane == 63) {
+        float* o = out + (size_t)item * 6;
+        o[0] = lo[0]; o[1] = lo[1]; o[2] = lo[2];
+        o[3] = hi[0]; o[4] = hi[1]; o[5] = hi[2];
+    }
 }
 
 hipError_t launch_src_bounds(const PairGeom& g, float* out, hipStream_t s) {
