@@ -135,7 +135,8 @@ struct Layout {
 // deferred-pixel flags, deferred-tile list and binning work list.
 struct RasterPlan {
     rvs_k::BatchDims d;
-    size_t status, counts, offsets, fill, lists, ranges, ktab, vbuf, imap, bsum, deferred, dtiles, work, tile_enc,
+    size_t zero_words;   // from status on, cleared before a launch set
+    size_t status, counts, offsets, fill, lists, ranges, ktab, vbuf, imap, deferred, dtiles, work, tile_enc,
         rbuf;
 };
 
@@ -187,9 +188,9 @@ void plan_raster(Layout& L, RasterPlan& R, int nsrc, int nviews, uint32_t ntiles
     const size_t nbins = (size_t)nsrc * ntiles;
     R.status = L.take(16 * sizeof(uint32_t));
     R.counts = L.take(nbins * sizeof(uint32_t));
+    R.fill = L.take(nbins * sizeof(uint32_t));   // status, counts and fill are cleared as one
+    R.zero_words = (L.o - R.status) / sizeof(uint32_t);
     R.offsets = L.take(nbins * sizeof(uint32_t));
-    R.fill = L.take(nbins * sizeof(uint32_t));
-    R.bsum = L.take(rvs_k::scan_blocks(nbins) * sizeof(unsigned long long));
     R.lists = L.take((size_t)d.cap * sizeof(uint32_t));
     R.ranges = L.take((size_t)d.range_cap * 256 * sizeof(uint32_t));
     R.ktab = L.take((size_t)d.range_cap * (1 + rvs_k::kBinTable) * sizeof(uint2));
@@ -204,10 +205,13 @@ void plan_raster(Layout& L, RasterPlan& R, int nsrc, int nviews, uint32_t ntiles
     R.tile_enc = L.take((size_t)ntiles);
     // the in-order replay's per-source results of its first rbuf_tiles tiles
     // (tiles beyond them take the one-block-per-tile replay): a sixty-fourth
-    // of the pixels, five floats per source
+    // of the pixels, five floats per source, or what fits 16 MB, if more (where
+    // sources and target are aligned every tile can be deferred: the VGA stereo
+    // pair's replay 141 -> 118 us).  Not in a fixed workspace.
     const uint64_t tile_px = (uint64_t)1 << (2 * shift);
+    const uint64_t small = keep_max > 0 ? 16 : (16ull << 20) / (tile_px * 20 * (uint64_t)nsrc);
     uint64_t rt = (uint64_t)npx / (64 * tile_px);
-    rt = rt < 16 ? 16 : rt;
+    rt = rt < small ? small : rt;
     // RVS_REPLAY_TILES=<n> lowers it (0: every deferred tile in order; the
     // results are the same)
     if (const char* env = std::getenv("RVS_REPLAY_TILES")) {
@@ -224,7 +228,6 @@ rvs_k::RasterWS carve_raster(char* base, const RasterPlan& R) {
     ws.counts = (uint32_t*)(base + R.counts);
     ws.offsets = (uint32_t*)(base + R.offsets);
     ws.fill = (uint32_t*)(base + R.fill);
-    ws.bsum = (unsigned long long*)(base + R.bsum);
     ws.lists = (uint32_t*)(base + R.lists);
     ws.ranges = (uint32_t*)(base + R.ranges);
     ws.ktab = (uint2*)(base + R.ktab);
@@ -236,13 +239,6 @@ rvs_k::RasterWS carve_raster(char* base, const RasterPlan& R) {
     ws.tile_enc = (uint8_t*)(base + R.tile_enc);
     ws.rbuf = (float*)(base + R.rbuf);
     return ws;
-}
-
-hipError_t reset_raster(const rvs_k::RasterWS& ws, const rvs_k::BatchDims& d, hipStream_t s) {
-    hipError_t e = rvs_k::launch_reset_u32(ws.status, 16, s);
-    if (e == hipSuccess) e = rvs_k::launch_reset_u32(ws.counts, (size_t)d.nsrc * d.ntiles, s);
-    if (e == hipSuccess) e = rvs_k::launch_reset_u32(ws.fill, (size_t)d.nsrc * d.ntiles, s);
-    return e;
 }
 
 // A view's tile grid and its place in the batch's global tile / pixel numbering.
@@ -279,14 +275,15 @@ void view_grid(rvs_k::ViewDesc& v, int w, int h, uint32_t& tiles, uint32_t& px, 
 
 // After a raster launch set: report list overflow (synchronises the stream).
 int check_raster_status(const rvs_k::RasterWS& ws, const rvs_k::BatchDims& d, uint32_t* needed_cap, hipStream_t s) {
-    uint32_t st[4];
+    uint32_t st[10];
     HIP_TRY(hipMemcpyAsync(st, ws.status, sizeof st, hipMemcpyDeviceToHost, s), "status copy");
     HIP_TRY(hipStreamSynchronize(s), "stream sync");
     if (st[1]) {
-        if (needed_cap) *needed_cap = st[2];
-        if (st[2] == 0xffffffffu)
+        const uint32_t entries = st[9] ? 0xffffffffu : st[8];   // saturated
+        if (needed_cap) *needed_cap = entries;
+        if (entries == 0xffffffffu)
             return fail(RVS_E_CAPACITY, "binned entries exceed 2^32 - 1: split the batch");
-        return fail(RVS_E_CAPACITY, "binned (quad, tile) entries %u exceed the list capacity %u", st[2], d.cap);
+        return fail(RVS_E_CAPACITY, "binned (quad, tile) entries %u exceed the list capacity %u", entries, d.cap);
     }
     return RVS_OK;
 }
@@ -485,8 +482,6 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
     PairGeom* dg = (PairGeom*)(base + P.geoms);
     ws = carve_raster(base, P.R);
     const rvs_k::BatchDims& d = P.R.d;
-    HIP_TRY(reset_raster(ws, d, s), "reset");
-    prof_mark(0, s);
     if (P.any_persp) {
         // culling tables: the source's resident one when it matches the views'
         // depth scale, else one built here; views with another depth scale do not cull
@@ -511,10 +506,14 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
             }
         }
     }
-    HIP_TRY(rvs_k::launch_upload(views.data(), views.size() * sizeof(rvs_k::ViewDesc), dviews, s), "view upload");
-    HIP_TRY(rvs_k::launch_upload(hg.data(), hg.size() * sizeof(PairGeom), dg, s), "geometry upload");
+    // views, then descriptors, as they lie in the workspace
+    std::vector<char> blob(P.geoms - P.views + hg.size() * sizeof(PairGeom));
+    std::memcpy(blob.data(), views.data(), views.size() * sizeof(rvs_k::ViewDesc));
+    std::memcpy(blob.data() + (P.geoms - P.views), hg.data(), hg.size() * sizeof(PairGeom));
+    HIP_TRY(rvs_k::launch_begin(blob.data(), blob.size(), dviews, ws.status, P.R.zero_words, s), "upload and reset");
+    prof_mark(0, s);
     if (!taps.empty())
-        HIP_TRY(rvs_k::launch_upload(taps.data(), taps.size() * sizeof(int2), rtab, s), "resize taps upload");
+        HIP_TRY(rvs_k::launch_begin(taps.data(), taps.size() * sizeof(int2), rtab, nullptr, 0, s), "resize taps upload");
     HIP_TRY(rvs_k::launch_bin<PairGeom>(dg, dviews, d, ws, s), "bin");
     prof_mark(1, s);
     HIP_TRY((rvs_k::launch_raster<PairGeom, rvs_k::MODE_BLEND>(dg, dviews, d, ws, s)), "raster");
@@ -757,9 +756,10 @@ int rvs_raster(const float* color, const float* depth, const float* uv, int in_w
     hg.rescale = rescale;
     rvs_k::ViewDesc* dv = (rvs_k::ViewDesc*)(base + ov);
     ArrayGeom* dg = (ArrayGeom*)(base + og);
-    HIP_TRY(rvs_k::launch_upload(&vd, sizeof vd, dv, s), "view upload");
-    HIP_TRY(rvs_k::launch_upload(&hg, sizeof hg, dg, s), "geometry upload");
-    HIP_TRY(reset_raster(ws, R.d, s), "reset");
+    std::vector<char> blob(og - ov + sizeof hg);
+    std::memcpy(blob.data(), &vd, sizeof vd);
+    std::memcpy(blob.data() + (og - ov), &hg, sizeof hg);
+    HIP_TRY(rvs_k::launch_begin(blob.data(), blob.size(), dv, ws.status, R.zero_words, s), "upload and reset");
     HIP_TRY(rvs_k::launch_bin<ArrayGeom>(dg, dv, R.d, ws, s), "bin");
     HIP_TRY((rvs_k::launch_raster<ArrayGeom, rvs_k::MODE_RAW>(dg, dv, R.d, ws, s)), "raster");
     HIP_TRY((rvs_k::launch_replay<ArrayGeom, rvs_k::MODE_RAW>(dg, dv, R.d, ws, s)), "replay");
@@ -798,8 +798,7 @@ int rvs_inpaint(float* color, const float* quality, int w, int h, void* workspac
     rvs_k::ViewDesc* dv = (rvs_k::ViewDesc*)workspace;
     const rvs_k::InpaintWS ws =
         rvs_k::inpaint_ws_carve((char*)workspace + align256(sizeof(rvs_k::ViewDesc)), (size_t)w * h, 1, w, h);
-    HIP_TRY(rvs_k::launch_reset_u32(ws.count, 1, s), "reset");
-    HIP_TRY(rvs_k::launch_upload(&vd, sizeof vd, dv, s), "view upload");
+    HIP_TRY(rvs_k::launch_begin(&vd, sizeof vd, dv, ws.count, 1, s), "view upload");
     HIP_TRY(rvs_k::launch_inpaint(dv, 1, w, h, ws, map_out, s), "inpaint");
     return RVS_OK;
 }
@@ -820,7 +819,7 @@ int rvs_resize_color(const float* src, int sw, int sh, float* dst, int dw, int d
     resize_taps(sh, dh, taps.data() + dw);
     hipStream_t s = (hipStream_t)stream;
     int2* dtaps = (int2*)workspace;
-    HIP_TRY(rvs_k::launch_upload(taps.data(), taps.size() * sizeof(int2), dtaps, s), "resize taps upload");
+    HIP_TRY(rvs_k::launch_begin(taps.data(), taps.size() * sizeof(int2), dtaps, nullptr, 0, s), "resize taps upload");
     HIP_TRY(rvs_k::launch_resize_color(src, sw, sh, dst, dw, dh, dtaps, s), "resize_color");
     return RVS_OK;
 }

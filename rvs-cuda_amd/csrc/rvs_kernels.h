@@ -86,7 +86,6 @@ struct RasterWS {
     float* vbuf;             // [range_cap work items][kItemFloats]: validities of triangles T1, T2 of the
                              // item's 256 quads, then its vertices [kBinQY + 1][kBinQX + 1][3] (u', v', depth)
     uint32_t* imap;          // [view][source][item] work index of a kept item, ~0 otherwise
-    unsigned long long* bsum;// scan block sums
     uint8_t* deferred;       // [global pixel] pixel handled by the in-order replay
     uint32_t* deferred_tiles;// [global tile]
     uint32_t* work;          // binning work items (view, source, block)
@@ -94,8 +93,8 @@ struct RasterWS {
                              // pixel (blending launches); written by every tile
     float* rbuf;             // [rbuf_tiles][source][tile pixel][5] the replay's per-source colour,
                              // depth and validity of deferred pixels
-    uint32_t* status;        // [0] n_deferred, [1] list overflow, [2] entries (saturated), [4] work items,
-                             // [5] inpainting tiles with holes
+    uint32_t* status;        // [0] n_deferred, [1] list overflow, [4] work items, [5] inpainting tiles with
+                             // holes, [8] [9] entries (64 bits)
 };
 
 struct BatchDims {
@@ -115,14 +114,12 @@ struct BatchDims {
 
 enum { MODE_BLEND = 0, MODE_RAW = 1 };
 
-hipError_t launch_reset_u32(uint32_t* p, size_t n, hipStream_t s);
 // Colour of every oversampled view resized to its encoded size (views[v].ecol);
 // views rasterised at their own size are skipped.
 hipError_t launch_resize_views(const ViewDesc* views, int nviews, int max_ew, int max_eh, hipStream_t s);
-// Scan blocks needed for nbins bins (bsum entries).
-size_t scan_blocks(size_t nbins);
-// Raw bytes into device memory through kernel arguments (stream-ordered, capturable).
-hipError_t launch_upload(const void* host, size_t bytes, void* dst, hipStream_t s);
+// Raw bytes (at least one) into device memory through kernel arguments, and `words`
+// words cleared (stream-ordered, capturable).
+hipError_t launch_begin(const void* host, size_t bytes, void* dst, uint32_t* zero, size_t words, hipStream_t s);
 
 // Binning blocks per row / column of a source grid.
 inline int bin_blocks_x(int sw) { return (sw - 1 + kBinQX - 1) / kBinQX; }
