@@ -153,6 +153,7 @@ void plan_raster(Layout& L, RasterPlan& R, int nsrc, int nviews, uint32_t ntiles
                  int n_unculled = 0, double culled_px_frac = 1.0) {
     rvs_k::BatchDims& d = R.d;
     d.nviews = nviews; d.nsrc = nsrc; d.ntiles = ntiles; d.npx = npx;
+    d.settle = 0;
     d.tile_shift = shift;
     // blocks of the passes over the kept items: items of equirectangular
     // targets differ widely in cost (those near a pole deal thousands of
@@ -481,6 +482,18 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
     rvs_k::ViewDesc* dviews = (rvs_k::ViewDesc*)(base + P.views);
     PairGeom* dg = (PairGeom*)(base + P.geoms);
     ws = carve_raster(base, P.R);
+    // Aligned cameras (no relative rotation, moved along an image axis: a
+    // rectified pair) map rows to rows or columns to columns, so that a plane
+    // facing them puts its pixels on the edges between quads, where both sides
+    // tie.  640x480 pair, replay: 118 us when the raster leaves all ties to it,
+    // 59 us (and 11 us more raster) when it settles them; 16 views from four
+    // panoramas lose 1 % of their time by looking for them.
+    for (const PairGeom& g : hg) {
+        const float I[9] = {1.f, 0.f, 0.f, 0.f, 1.f, 0.f, 0.f, 0.f, 1.f};
+        bool same = !g.src_erp && !g.dst_erp && g.t[0] == 0.f && (g.t[1] == 0.f || g.t[2] == 0.f);
+        for (int k = 0; k < 9; ++k) same = same && g.R[k] == I[k];
+        if (same) P.R.d.settle = 1;
+    }
     const rvs_k::BatchDims& d = P.R.d;
     if (P.any_persp) {
         // culling tables: the source's resident one when it matches the views'

@@ -34,7 +34,10 @@ constexpr int kBinBlocks = 2048;    // persistent binning blocks (work items pas
 constexpr int kFlatBlocks = 65536;  // persistent blocks of the passes over the kept work items
 constexpr int kRasterGroup = 4;     // sources rasterised together in k_raster's one-phase instantiation
 constexpr int kRasterGroupMulti = 4; // sources per phase of the looping instantiation (more sources)
-constexpr int kRasterCache = 1536;  // binned quads per phase whose coverage-pass results stay in LDS
+// binned quads per phase whose coverage-pass results stay in LDS; with the queue below a block of the
+// looping instantiation takes 20 KB, so 7 waves per SIMD fit (1536 and 500: 6; an 8192x4096
+// panorama of eleven, three scenes, raster ms 7.7 13.7 9.0 -> 7.5 11.6 8.6)
+constexpr int kRasterCache = 960;
 constexpr int kRasterCacheOne = 960; // the same for launch sets of up to kRasterGroup sources (one phase)
 // k_raster: a triangle with more pixels of a tile than this in its box is shared by the lanes of a
 // wave.  16 views of mixed sizes / an 8192x4096 equirectangular view, two scenes each, raster ms: 32
@@ -43,7 +46,7 @@ constexpr int kRasterCacheOne = 960; // the same for launch sets of up to kRaste
 // a pole: side by side is as good there until they exceed a wave).
 constexpr int kWidePx = 64;
 constexpr int kWideQueueOne = 100;  // such triangles put off per phase (in the LDS the one-phase blocks leave free)
-constexpr int kWideQueue = 500;     // the same in the looping instantiation
+constexpr int kWideQueue = 100;     // the same in the looping instantiation
 constexpr int kMaxSourceSide = 65536;  // bins hold quads as (row << 16) | column; also the
                                        // largest target side (tile coordinates fit 16 bits)
 constexpr int kFallbackBlocks = 1024;
@@ -109,6 +112,8 @@ struct BatchDims {
                              // 5 (32 x 32, 1024-thread blocks)
     uint32_t flat_blocks;    // blocks of the passes over the kept work items
     uint32_t rbuf_tiles;     // deferred tiles whose sources are replayed in parallel (RasterWS::rbuf)
+    uint32_t settle;         // exact ties are expected: the raster settles them (MODE_BLEND, up to
+                             // kRasterGroup sources)
     uint32_t kept_geom;      // kept work items also store vertex windows and validities (vbuf)
 };
 

@@ -1007,8 +1007,13 @@ constexpr uint32_t kDeferKey = 0xffffffffu;
 
 // Pushes candidate `id` of triangle T for the tile's pixel p with centre (fx,
 // fy): the exact coverage test, then the key updates.  r: recip(T.den).
-__device__ __forceinline__ void raster_push(const Tri& T, float r, bool special, uint32_t id, float fx, float fy, int p,
-                                            unsigned long long* key1, uint32_t* key2) {
+// Sets *tie (if any) when it meets a candidate of the same score.
+// TIES: the second pass, over tied pixels only (their shape in tie[p], 0 for the
+// others; their depth's bits in key2[p]): see settle_ties.
+template <bool TIES>
+__device__ __forceinline__ void raster_push(const Tri& T, float r, bool special, uint32_t id, uint32_t ij, float fx,
+                                            float fy, int p, unsigned long long* key1, uint32_t* key2, float* tie) {
+    if (TIES && !(tie[p] > 0.f)) return;
     // tri_num at the pixel
     const float dx = fx - T.C0, dy = fy - T.C1;
     const float n1 = (T.B1 - T.C1) * dx + (T.C0 - T.B0) * dy, n2 = (T.C1 - T.A1) * dx + (T.A0 - T.C0) * dy;
@@ -1018,9 +1023,20 @@ __device__ __forceinline__ void raster_push(const Tri& T, float r, bool special,
     // the score only orders candidates outside the ambiguity band:
     // v_rcp_f32 (1 ulp) keeps its error within 5 * 2^-24 relative
     const float f = T.tv * __builtin_amdgcn_rcpf(dd * dd * dd);
+    if (TIES) {
+        const float v = tie[p], w = u2f(key2[p]);
+        if (!special && f2u(dd) == f2u(w) && T.tv == v) {
+            atomicMin(&key1[p], ((unsigned long long)ij << 32) | ((unsigned long long)(id & 3u) << 30) | (id >> 2));
+        } else {
+            const float fw = v * __builtin_amdgcn_rcpf(w * w * w);
+            if (special || !(f < fw - fw * RVS_AMBIGUITY)) atomicMin(&key1[p], 0ull);
+        }
+        return;
+    }
     const bool defer = special || !depth_regular(dd);
     const unsigned long long k = defer ? 0ull : ((unsigned long long)f2u(f) << 32) | id;
     const unsigned long long old = atomicMax(&key1[p], k);
+    if (tie && (uint32_t)(old >> 32) == f2u(f)) *tie = 1.f;
     // the candidate that is not (or no longer) the maximum goes to the runner-up slot
     atomicMax(&key2[p], defer ? kDeferKey : (uint32_t)((old < k ? old : k) >> 32));
 }
@@ -1060,10 +1076,10 @@ __device__ __forceinline__ bool take_validity(Tri& T, float rescale, float tv_kn
 // it changes nothing).  A finite triangle with more than kWidePx pixels of the
 // tile in its box is left to raster_wide while the queue Q (null: none) has
 // room.
-template <int TILE, bool KNOWN, class Queue>
-__device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_t id, bool prol_false_possible, int tx0,
+template <int TILE, bool KNOWN, bool TIES, class Queue>
+__device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_t id, uint32_t ij, bool prol_false_possible, int tx0,
                                    int ty0, int out_w, int out_h, float rescale, unsigned long long* key1,
-                                   uint32_t* key2, bool undecided, float tv_known, Queue* Q) {
+                                   uint32_t* key2, bool undecided, float tv_known, Queue* Q, float* tie) {
     Tri T;
     tri_load(T, a, b, c);
     int xa, xb, ya, yb;
@@ -1072,6 +1088,7 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
     // a finite den has finite image coordinates
     bool special = !is_finite(a.z + b.z + c.z) || !is_finite(T.den) || (prol_false_possible && !prol) || undecided;
     if (!cover_den(T.den)) {
+        if (TIES) return;   // done in the first pass
         // degenerate, gigantic or non-finite: whatever it may cover is deferred
         for (int y = ya; y <= yb; ++y)
             for (int x = xa; x <= xb; ++x) {
@@ -1120,7 +1137,7 @@ __device__ __forceinline__ void raster_tri(float3 a, float3 b, float3 c, uint32_
             while (mask) {
                 const int bit = __builtin_ctz(mask), col = bit & 7, row = bit >> 3;
                 mask &= mask - 1u;
-                raster_push(T, r, special, id, fx0 + (float)col, fy0 + (float)row, p0 + row * TILE + col, key1, key2);
+                raster_push<TIES>(T, r, special, id, ij, fx0 + (float)col, fy0 + (float)row, p0 + row * TILE + col, key1, key2, tie);
             }
         }
 }
@@ -1153,20 +1170,20 @@ static_assert(kRasterGroup == 4 && kRasterGroupMulti == 4, "a phase of four sour
 // bins: stretched across a depth edge, magnified, or near a pole.
 // Measured: two 3840x2160 views of 11 perspective sources, raster 4.03 -> 3.40
 // ms; 8 views of 1920x1080 of four panoramas 1.80 -> 1.22 ms.
-template <int TILE, int NT, bool KEPT, class G, class Queue>
+template <int TILE, int NT, bool KEPT, bool TIES, class G, class Queue>
 __device__ __forceinline__ void raster_wide(const G* gv, const Phase& ph, uint32_t nwide, const Queue& Q, int wave, int tx0, int ty0, int out_w,
                                             int out_h, unsigned long long (*key1)[NT], uint32_t (*key2)[NT],
-                                            const RasterWS& ws, const BatchDims& d, uint32_t vs0) {
+                                            const RasterWS& ws, const BatchDims& d, uint32_t vs0,
+                                            float (*ties)[NT], float* tie) {
     constexpr uint32_t NW = NT / 64;
     for (uint32_t q0 = (uint32_t)wave; q0 < nwide; q0 += 64u * NW) {
         const uint32_t q = q0 + NW * (uint32_t)lane_now();
         Tri T;
         float tr = 0.f;
         int k = 0, xa = 0, xb = -1, ya = 0, yb = -1, sp = 0;
-        uint32_t id = 0u;
+        uint32_t id = 0u, code = 0u;
         if (q < nwide) {
             id = Q.id[q];
-            uint32_t code;
             k = ph.find(ws, id >> 2, code);
             int i, j;
             unpack_ij(code, i, j);
@@ -1202,6 +1219,7 @@ __device__ __forceinline__ void raster_wide(const G* gv, const Phase& ph, uint32
             const int bw = __builtin_amdgcn_readlane(xb, l) - wx + 1;
             const int n = bw * (__builtin_amdgcn_readlane(yb, l) - wy + 1);
             const int sk = __builtin_amdgcn_readlane(k | sp, l);
+            const uint32_t wij = TIES ? (uint32_t)__builtin_amdgcn_readlane((int)code, l) : 0u;
             const uint32_t wid = (uint32_t)__builtin_amdgcn_readlane((int)id, l);
             const float inv = __builtin_amdgcn_rcpf((float)bw), r = lane_f(tr, l);
             for (int i = lane_now(); i < n; i += 64) {
@@ -1211,8 +1229,9 @@ __device__ __forceinline__ void raster_wide(const G* gv, const Phase& ph, uint32
                 float n1, n2;
                 tri_num(W, x, y, n1, n2);
                 if (!tri_outside_r(r, n1, n2))
-                    raster_push(W, r, sk >= 0x100, wid, (float)x + 0.5f, (float)y + 0.5f,
-                                (y - ty0) * TILE + (x - tx0), key1[sk & 0xff], key2[sk & 0xff]);
+                    raster_push<TIES>(W, r, sk >= 0x100, wid, wij, (float)x + 0.5f, (float)y + 0.5f,
+                                (y - ty0) * TILE + (x - tx0), key1[sk & 0xff], key2[sk & 0xff],
+                                      TIES ? ties[sk & 0xff] : tie);
             }
         }
     }
@@ -1235,10 +1254,11 @@ struct RasterCache {
 // scores are deferred to the in-order replay.
 // gt: any descriptor of the view (target-side fields: the same for all its
 // sources, so they are read once per wave).
-template <int TILE, bool KEPT, class G, class Cache, class Queue>
+template <int TILE, bool KEPT, bool TIES, class G, class Cache, class Queue>
 __device__ __forceinline__ void raster_quad(const G& g, const G& gt, uint32_t ij, uint32_t e, int tx0, int ty0,
                                             int out_w, int out_h, unsigned long long* key1, uint32_t* key2, Cache* C,
-                                            Queue* Q, const RasterWS& ws, const BatchDims& d, uint32_t vs) {
+                                            Queue* Q, const RasterWS& ws, const BatchDims& d, uint32_t vs,
+                                            float* tie) {
     int i, j;
     unpack_ij(ij, i, j);
     const uint32_t wi = kept_index<KEPT>(ws, d, vs, ij);
@@ -1261,10 +1281,11 @@ __device__ __forceinline__ void raster_quad(const G& g, const G& gt, uint32_t ij
     const bool gate = v01.z > 0.f && v10.z > 0.f && v01.x > 0.f && v10.x > 0.f;
     const uint32_t s0 = e << 2;
     if (gate && v00.z > 0.f && v00.x > 0.f)
-        raster_tri<TILE, KEPT>(v00, v01, v10, s0, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und, tvk.x, Q);
+        raster_tri<TILE, KEPT, TIES>(v00, v01, v10, s0, ij, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und, tvk.x, Q,
+                                     tie);
     if (gate && v11.z > 0.f && v11.x > 0.f)
-        raster_tri<TILE, KEPT>(v11, v10, v01, s0 | 1u, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und,
-                               tvk.y, Q);
+        raster_tri<TILE, KEPT, TIES>(v11, v10, v01, s0 | 1u, ij, false, tx0, ty0, out_w, out_h, gt.rescale, key1, key2, und,
+                               tvk.y, Q, tie);
     if (__builtin_expect(gate && gt.wrap && j == 0, 0)) {
         float3 l[2];
         if (KEPT) kept_seam(ws, d, vs, i, g.sw, l);
@@ -1272,8 +1293,8 @@ __device__ __forceinline__ void raster_quad(const G& g, const G& gt, uint32_t ij
 #pragma unroll 1
         for (uint32_t k = 0; k < 2u; ++k) {
             const bool s3 = k != 0u;
-            raster_tri<TILE, false>(s3 ? v10 : l[0], s3 ? l[1] : v00, s3 ? v00 : l[1], s0 | (2u + k), true, tx0, ty0,
-                                    out_w, out_h, gt.rescale, key1, key2, und, 0.f, (Queue*)nullptr);
+            raster_tri<TILE, false, TIES>(s3 ? v10 : l[0], s3 ? l[1] : v00, s3 ? v00 : l[1], s0 | (2u + k), ij, true, tx0, ty0,
+                                    out_w, out_h, gt.rescale, key1, key2, und, 0.f, (Queue*)nullptr, tie);
         }
     }
     if (C) {
@@ -1346,6 +1367,7 @@ struct RasterLds {
     RasterCache<(MULTI ? kRasterCache : kRasterCacheOne) * AREA> cache;
     typedef WideQueue<(MULTI ? kWideQueue : kWideQueueOne) * AREA> Queue;
     Queue wide;
+    float s_tie;          // two candidates of one score met (0 / 1)
 };
 
 // One tile of k_raster.  Bound by the issue of VALU instructions (0.62 T/s of wave
@@ -1362,7 +1384,7 @@ struct RasterLds {
 // window and validities (nearly always), so this code evaluates no vertex and
 // no validity of slots 0 and 1: a third of the instructions of the general
 // form, whose registers would otherwise spill around them.
-template <class G, int MODE, bool MULTI, int TILE, bool KEPT>
+template <class G, int MODE, bool MULTI, int TILE, bool KEPT, bool SETTLE>
 __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
                                             const BatchDims& d, const RasterWS& ws, RasterLds<MULTI, TILE>& L) {
     typedef RasterLds<MULTI, TILE> Lds;
@@ -1374,6 +1396,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
     Queue& wide = L.wide;
     int& s_deferred = L.s_deferred;
     int& s_hole = L.s_hole;
+    float& s_tie = L.s_tie;
     const uint32_t T = tile_of_block(blockIdx.x, d.ntiles);
     if (T >= d.ntiles) return;
     const int v = find_view(views, d.nviews, T);
@@ -1398,6 +1421,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
         if (tid == 0) {
             if (s0 == 0) { s_deferred = 0; s_hole = 0; }
             wide.n = 0u;
+            if (SETTLE) s_tie = 0.f;
         }
         uint32_t end[GRP], add[GRP], acc = 0u;
 #pragma unroll
@@ -1411,7 +1435,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
         const Phase ph = {end[0], end[1], end[2], acc, add[0], add[1] - add[0], add[2] - add[1], add[3] - add[2]};
         __syncthreads();
         const uint32_t N = ph.n;
-        const bool cached = N <= (uint32_t)cache.cap;
+        bool cached = N <= (uint32_t)cache.cap;
         // a wave-uniform trip count; the entry index is re-derived each trip
         const uint32_t trips = (N + (uint32_t)NT - 1u) / (uint32_t)NT;
         for (uint32_t it = 0; it < trips; ++it) {
@@ -1419,15 +1443,82 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
             if (e >= N) continue;
             uint32_t ij;
             const int k = ph.find(ws, e, ij);
-            raster_quad<TILE, KEPT>(gv[s0 + k], gv[0], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k], cached ? &cache : nullptr,
-                              &wide, ws, d, (uint32_t)(v * d.nsrc + s0 + k));
+            raster_quad<TILE, KEPT, false>(gv[s0 + k], gv[0], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k],
+                                           cached ? &cache : nullptr, &wide, ws, d, (uint32_t)(v * d.nsrc + s0 + k),
+                                           SETTLE ? &s_tie : (float*)nullptr);
         }
         __syncthreads();
         const uint32_t nwide = __builtin_amdgcn_readfirstlane(min(wide.n, Queue::cap));
         if (nwide) {   // the same in every wave
-            raster_wide<TILE, NT, KEPT>(gv + s0, ph, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1,
-                                  key2, ws, d, (uint32_t)(v * d.nsrc + s0));
+            raster_wide<TILE, NT, KEPT, false>(gv + s0, ph, nwide, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1, key2,
+                                               ws, d, (uint32_t)(v * d.nsrc + s0), (float(*)[NT])nullptr,
+                                               SETTLE ? &s_tie : (float*)nullptr);
             __syncthreads();
+        }
+        if (SETTLE && __builtin_amdgcn_readfirstlane(f2u(s_tie)) != 0u) {
+            // Settles exact ties (a plane seen from an aligned camera puts every
+            // pixel on the edge between two quads): where all candidates within
+            // the ambiguity of the best have its very depth and validity, the
+            // fold keeps the first of them -- each later one meets a ratio of 1
+            // and its own validity -- so a second pass takes the least
+            // (quad, slot); any other candidate that near leaves the pixel
+            // deferred.  The second pass replaces the replay of those pixels:
+            // 640x480 pair 290 -> 245 us.
+            auto ties = reinterpret_cast<float(*)[NT]>(&cache);   // the cache is given up
+            static_assert(sizeof(cache) >= sizeof(float) * GRP * NT, "the ties' shapes fit the cache");
+            const int t2 = wave_base + lane_now();
+            const int px = tx0 + (t2 % TILE), py = ty0 + (t2 / TILE);
+            float shape[GRP];
+#pragma unroll
+            for (int k = 0; k < GRP; ++k) {
+                shape[k] = 0.f;
+                if (k >= gs) continue;
+                const unsigned long long kw = key1[k][t2];
+                if (kw == 0ull || key2[k][t2] != (uint32_t)(kw >> 32) || ((uint32_t)kw & 2u)) continue;
+                uint32_t ij;
+                ph.find(ws, (uint32_t)kw >> 2, ij);
+                const KeptQuad kq = kept_quad(ws, kept_index<true>(ws, d, (uint32_t)(v * d.nsrc + s0 + k), ij), ij);
+                const int slot = (int)((uint32_t)kw & 1u);
+                float3 c3[3];
+                kept_corners(kq.v, slot, c3);
+                Tri W;
+                tri_load(W, c3[0], c3[1], c3[2]);
+                float l1, l2, l3;
+                tri_bary(W, px, py, l1, l2, l3);
+                shape[k] = kq.tv[slot];
+                key1[k][t2] = ~0ull;
+                key2[k][t2] = f2u(tri_depth(W, l1, l2, l3));
+            }
+            if (t2 == 0) wide.n = 0u;
+            __syncthreads();   // the cache and the queue are no longer read
+#pragma unroll
+            for (int k = 0; k < GRP; ++k) ties[k][t2] = shape[k];
+            __syncthreads();
+            for (uint32_t it = 0; it < trips; ++it) {
+                const uint32_t e = it * (uint32_t)NT + (uint32_t)(wave_base + lane_now());
+                if (e >= N) continue;
+                uint32_t ij;
+                const int k = ph.find(ws, e, ij);
+                raster_quad<TILE, KEPT, true>(gv[s0 + k], gv[0], ij, e, tx0, ty0, vd.w, vd.h, key1[k], key2[k],
+                                              (decltype(&cache))nullptr, &wide, ws, d,
+                                              (uint32_t)(v * d.nsrc + s0 + k), ties[k]);
+            }
+            __syncthreads();
+            const uint32_t nw = __builtin_amdgcn_readfirstlane(min(wide.n, Queue::cap));
+            if (nw) {
+                raster_wide<TILE, NT, KEPT, true>(gv + s0, ph, nw, wide, wave_base / 64, tx0, ty0, vd.w, vd.h, key1, key2,
+                                                  ws, d, (uint32_t)(v * d.nsrc + s0), ties, &s_tie);
+                __syncthreads();
+            }
+            const int t4 = wave_base + lane_now();
+            for (int k = 0; k < gs; ++k) {
+                if (!(ties[k][t4] > 0.f)) continue;
+                const unsigned long long o = key1[k][t4];
+                const uint32_t id = ((uint32_t)o << 2) | ((uint32_t)o >> 30);
+                key1[k][t4] = (1ull << 32) | id;
+                key2[k][t4] = o == 0ull || o == ~0ull ? kDeferKey : 0u;
+            }
+            cached = false;
         }
         const int t2 = wave_base + lane_now();
         const int px = tx0 + (t2 % TILE), py = ty0 + (t2 / TILE);
@@ -1526,15 +1617,17 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
 // free of the blend state's registers.
 // TILE: the tile edge; a block has a thread per pixel (256 or 1024 threads),
 // and the caches scale with the tile's area.
-template <class G, int MODE, bool MULTI, int TILE>
-__global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_eu(MULTI ? (TILE > kTile ? 4 : 6) : 8)))
+// SETTLE: exact ties are settled here (BatchDims::settle; one phase only).  Where
+// ties are chance, meeting them costs the candidate loop more than their replay.
+template <class G, int MODE, bool MULTI, int TILE, bool SETTLE>
+__global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_eu(MULTI ? (TILE > kTile ? 4 : 7) : 8)))
 k_raster(const G* __restrict__ geoms, const ViewDesc* __restrict__ views, BatchDims d, RasterWS ws) {
     __shared__ RasterLds<MULTI, TILE> lds;
     if (ws.status[1]) return;   // bins not filled: capacity reported to the host
     if (d.kept_geom && ws.status[4] <= d.range_cap)   // the same for the whole launch
-        raster_tile<G, MODE, MULTI, TILE, true>(geoms, views, d, ws, lds);
+        raster_tile<G, MODE, MULTI, TILE, true, SETTLE>(geoms, views, d, ws, lds);
     else
-        raster_tile<G, MODE, MULTI, TILE, false>(geoms, views, d, ws, lds);
+        raster_tile<G, MODE, MULTI, TILE, false, false>(geoms, views, d, ws, lds);
 }
 
 // ------------------------------------------------------ in-order replay
@@ -1906,20 +1999,17 @@ __global__ void __launch_bounds__(256) k_fallback_blend(const ViewDesc* __restri
 template <class G, int MODE>
 hipError_t launch_raster(const G* geoms, const ViewDesc* views, const BatchDims& d, const RasterWS& ws,
                          hipStream_t s) {
-    const unsigned blocks = 8u * ((d.ntiles + 7u) / 8u);
-    const bool multi = d.nsrc > kRasterGroup;
-    if (d.tile_shift == 5) {
-        constexpr int NT = kTileBig * kTileBig;
-        if (multi)
-            hipLaunchKernelGGL((k_raster<G, MODE, true, kTileBig>), dim3(blocks), dim3(NT), 0, s, geoms, views, d, ws);
-        else
-            hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig>), dim3(blocks), dim3(NT), 0, s, geoms, views, d, ws);
+    const dim3 blocks(8u * ((d.ntiles + 7u) / 8u)), nb(kTileBig * kTileBig), nt(kTile * kTile);
+    const bool big = d.tile_shift == 5;
+    if (d.nsrc > kRasterGroup) {
+        if (big) hipLaunchKernelGGL((k_raster<G, MODE, true, kTileBig, false>), blocks, nb, 0, s, geoms, views, d, ws);
+        else hipLaunchKernelGGL((k_raster<G, MODE, true, kTile, false>), blocks, nt, 0, s, geoms, views, d, ws);
+    } else if (d.settle) {
+        if (big) hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig, true>), blocks, nb, 0, s, geoms, views, d, ws);
+        else hipLaunchKernelGGL((k_raster<G, MODE, false, kTile, true>), blocks, nt, 0, s, geoms, views, d, ws);
     } else {
-        constexpr int NT = kTile * kTile;
-        if (multi)
-            hipLaunchKernelGGL((k_raster<G, MODE, true, kTile>), dim3(blocks), dim3(NT), 0, s, geoms, views, d, ws);
-        else
-            hipLaunchKernelGGL((k_raster<G, MODE, false, kTile>), dim3(blocks), dim3(NT), 0, s, geoms, views, d, ws);
+        if (big) hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig, false>), blocks, nb, 0, s, geoms, views, d, ws);
+        else hipLaunchKernelGGL((k_raster<G, MODE, false, kTile, false>), blocks, nt, 0, s, geoms, views, d, ws);
     }
     return hipGetLastError();
 }
