@@ -107,15 +107,19 @@ class Server:
         if n < 0:
             raise RuntimeError("no output kept for request %d" % k)
         out = _new_bytes(None, n)   # not yet seen by anyone else, so it may be written
-        _lib().rvs_server_output(self.h, int(k), _bytes_at(out), n)
+        if _lib().rvs_server_output(self.h, int(k), _bytes_at(out), n) != n:   # another run replaced it meanwhile
+            raise RuntimeError("output of request %d changed while it was read" % k)
         return out
 
 
 # An uninitialised bytes object and its buffer: one copy of an output instead
-# of a zeroed array, a copy into it and a copy out of it.
-_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+# of a zeroed array, a copy into it and a copy out of it.  The function objects
+# are this module's own: those of C.pythonapi are shared by the whole process,
+# and so are their prototypes.
+_python = C.PyDLL(None)
+_new_bytes = _python.PyBytes_FromStringAndSize
 _new_bytes.argtypes, _new_bytes.restype = [C.c_char_p, C.c_ssize_t], C.py_object
-_bytes_at = C.pythonapi.PyBytes_AsString
+_bytes_at = _python.PyBytes_AsString
 _bytes_at.argtypes, _bytes_at.restype = [C.py_object], C.c_void_p
 
 
