@@ -495,6 +495,7 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
         if (same) P.R.d.settle = 1;
     }
     const rvs_k::BatchDims& d = P.R.d;
+    prof_mark(0, s);   // binning starts with what a call builds or uploads for it
     if (P.any_persp) {
         // culling tables: the source's resident one when it matches the views'
         // depth scale, else one built here; views with another depth scale do not cull
@@ -524,7 +525,6 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
     std::memcpy(blob.data(), views.data(), views.size() * sizeof(rvs_k::ViewDesc));
     std::memcpy(blob.data() + (P.geoms - P.views), hg.data(), hg.size() * sizeof(PairGeom));
     HIP_TRY(rvs_k::launch_begin(blob.data(), blob.size(), dviews, ws.status, P.R.zero_words, s), "upload and reset");
-    prof_mark(0, s);
     if (!taps.empty())
         HIP_TRY(rvs_k::launch_begin(taps.data(), taps.size() * sizeof(int2), rtab, nullptr, 0, s), "resize taps upload");
     HIP_TRY(rvs_k::launch_bin<PairGeom>(dg, dviews, d, ws, s), "bin");
