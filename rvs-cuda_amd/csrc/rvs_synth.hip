@@ -255,10 +255,14 @@ __global__ void __launch_bounds__(256) k_src_bounds(PairGeom g, int bins_x, int 
     const float inf = __builtin_inff();
     float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     // points in pairs; the minima pass over NaNs, and a point with any
-    // non-finite coordinate becomes NaNs
+    // non-finite coordinate becomes NaNs (times 0 it gives a NaN; a plain sum
+    // of finite coordinates can overflow)
+    auto finite = [](float3 p) {
+        return __builtin_fmaf(p.z, 0.f, __builtin_fmaf(p.y, 0.f, p.x * 0.f)) == 0.f;
+    };
     auto add = [&](float3 p, float3 q) {
         const float n = __builtin_nanf("");
-        const bool a = is_finite(p.x + p.y + p.z), b = is_finite(q.x + q.y + q.z);
+        const bool a = finite(p), b = finite(q);
         const float ps[3] = {a ? p.x : n, a ? p.y : n, a ? p.z : n}, qs[3] = {b ? q.x : n, b ? q.y : n, b ? q.z : n};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
