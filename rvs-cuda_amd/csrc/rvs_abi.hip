@@ -298,9 +298,13 @@ struct SynthPlan {
     size_t views, geoms, bounds, quality, color, inpaint, resized, rtab, total;
     int tile_shift;       // log2 of the launch set's tile edge
     int max_w, max_h;     // largest raster (oversampled by Precision)
+    size_t hole_tiles;    // inpainting tiles of all views
     int max_ew, max_eh;   // largest view
     bool any_persp, any_erp, any_rescaled;
 };
+
+// Inpainting tiles of a w x h raster.
+size_t hole_tiles(int w, int h) { return (size_t)rvs_k::inpaint_tiles(w) * rvs_k::inpaint_tiles(h); }
 
 // Raster size of a view with Precision `rescale` (SynthesizedView.cpp:326-329).
 void raster_size(const rvs_cam& c, float rescale, int& w, int& h) {
@@ -320,7 +324,7 @@ int plan_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int n_
     }
     uint64_t tiles = 0, px = 0, rpx = 0, persp_px = 0, rtaps = 0;
     int n_erp = 0;   // equirectangular targets: their work items are not culled
-    P.max_w = 0; P.max_h = 0; P.max_ew = 0; P.max_eh = 0; P.any_persp = false; P.any_erp = false;
+    P.max_w = 0; P.max_h = 0; P.hole_tiles = 0; P.max_ew = 0; P.max_eh = 0; P.any_persp = false; P.any_erp = false;
     P.any_rescaled = false;
     // the launch set's tile edge: the largest any view asks for
     int shift = 4;
@@ -358,6 +362,7 @@ int plan_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int n_
         }
         tiles += (uint64_t)((rw + edge - 1) / edge) * ((rh + edge - 1) / edge);
         px += (uint64_t)rw * rh;
+        P.hole_tiles += hole_tiles(rw, rh);
     }
     if (max_sw > rvs_k::kMaxSourceSide || max_sh > rvs_k::kMaxSourceSide)
         return fail(RVS_E_UNSUPPORTED, "synthesize: source side above %d", rvs_k::kMaxSourceSide);
@@ -378,20 +383,22 @@ int plan_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int n_
     P.color = L.take((size_t)px * 3 * sizeof(float));
     plan_raster(L, P.R, n_src, n_views, (uint32_t)tiles, (uint32_t)px, cap, max_sw, max_sh, keep_max, shift,
                 P.any_erp, n_erp, px ? (double)persp_px / (double)px : 1.0);
-    P.inpaint = L.take(rvs_k::inpaint_ws_bytes((size_t)px, n_views, P.max_w, P.max_h));
+    P.inpaint = L.take(rvs_k::inpaint_ws_bytes((size_t)px, P.hole_tiles));
     // oversampled views: their colour resized to the view's size, for the encoder
     P.resized = L.take((size_t)rpx * 3 * sizeof(float));
     P.rtab = L.take((size_t)rtaps * sizeof(int2));   // their resize taps
     P.total = L.o;
     if (views) {
         views->resize(n_views);
-        uint32_t tb = 0, pb = 0;
+        uint32_t tb = 0, pb = 0, hb = 0;
         for (int v = 0; v < n_views; ++v) {
             rvs_k::ViewDesc& d = (*views)[v];
             std::memset(&d, 0, sizeof d);
             int rw, rh;
             raster_size(tgts[v].cam, tgts[v].rescale, rw, rh);
             view_grid(d, rw, rh, tb, pb, shift);
+            d.hole_base = hb;
+            hb += (uint32_t)hole_tiles(rw, rh);
             d.ew = tgts[v].cam.w;
             d.eh = tgts[v].cam.h;
             d.bitdepth = tgts[v].bitdepth;
@@ -542,7 +549,7 @@ int enqueue_synth(const rvs_source* srcs, int n_src, const rvs_target* tgts, int
         HIP_TRY(hipStreamWaitEvent(sf, split_ev, 0), "split wait");
         s = sf;
     }
-    rvs_k::InpaintWS iws = rvs_k::inpaint_ws_carve(base + P.inpaint, d.npx, n_views, P.max_w, P.max_h);
+    rvs_k::InpaintWS iws = rvs_k::inpaint_ws_carve(base + P.inpaint, d.npx, P.hole_tiles);
     iws.count = ws.status + 5;  // zeroed with the launch set's status
     iws.rflags = ws.tile_enc;   // tiles the raster left without holes or deferred pixels are skipped
     HIP_TRY(rvs_k::launch_inpaint(dviews, n_views, P.max_w, P.max_h, iws, nullptr, s), "inpaint");
@@ -793,7 +800,7 @@ int rvs_blend_step(float* acc_color, float* acc_quality, float* acc_depth, float
 
 size_t rvs_inpaint_workspace_size(int w, int h) {
     if (w < 1 || h < 1) return 0;
-    return align256(sizeof(rvs_k::ViewDesc)) + align256(rvs_k::inpaint_ws_bytes((size_t)w * h, 1, w, h));
+    return align256(sizeof(rvs_k::ViewDesc)) + align256(rvs_k::inpaint_ws_bytes((size_t)w * h, hole_tiles(w, h)));
 }
 
 int rvs_inpaint(float* color, const float* quality, int w, int h, void* workspace, size_t ws_bytes, int32_t* map_out,
@@ -810,7 +817,7 @@ int rvs_inpaint(float* color, const float* quality, int w, int h, void* workspac
     vd.quality = (float*)quality;
     rvs_k::ViewDesc* dv = (rvs_k::ViewDesc*)workspace;
     const rvs_k::InpaintWS ws =
-        rvs_k::inpaint_ws_carve((char*)workspace + align256(sizeof(rvs_k::ViewDesc)), (size_t)w * h, 1, w, h);
+        rvs_k::inpaint_ws_carve((char*)workspace + align256(sizeof(rvs_k::ViewDesc)), (size_t)w * h, hole_tiles(w, h));
     HIP_TRY(rvs_k::launch_begin(&vd, sizeof vd, dv, ws.count, 1, s), "view upload");
     HIP_TRY(rvs_k::launch_inpaint(dv, 1, w, h, ws, map_out, s), "inpaint");
     return RVS_OK;

@@ -124,14 +124,24 @@ struct HoleTile {
     int t, v, tx0, ty0;
 };
 
-__device__ inline HoleTile tile_place(const InpaintWS& ws, int t) {
+__device__ inline HoleTile tile_place(const ViewDesc* views, int t, int v) {
     HoleTile H;
     H.t = t;
-    H.v = t / ws.tpv;
-    const int r = t - H.v * ws.tpv;
-    H.tx0 = (r % ws.ttx) * kInpTile;
-    H.ty0 = (r / ws.ttx) * kInpTile;
+    H.v = v;
+    const int r = t - (int)views[v].hole_base, across = inpaint_tiles(views[v].w);
+    H.tx0 = (r % across) * kInpTile;
+    H.ty0 = (r / across) * kInpTile;
     return H;
+}
+
+// View of tile t (views are sorted by hole_base).
+__device__ inline int tile_view(const ViewDesc* views, int nviews, int t) {
+    int lo = 0, hi = nviews - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if ((int)views[mid].hole_base <= t) lo = mid; else hi = mid - 1;
+    }
+    return lo;
 }
 
 // ---------------------------------------------------------------- kernels
@@ -147,12 +157,11 @@ __device__ inline bool not_known(const ViewDesc& vd, const InpaintWS& ws, int x,
     return !(vd.quality[(size_t)y * vd.w + x] > 0.f);
 }
 
-// Whether tile t may hold a hole, from the raster's tile flags.
-__device__ inline bool may_have_hole(const ViewDesc* views, const InpaintWS& ws, int t) {
-    const HoleTile H = tile_place(ws, t);
-    const ViewDesc& vd = views[H.v];
-    if (H.tx0 >= vd.w || H.ty0 >= vd.h) return false;
+// Whether tile t of view v may hold a hole, from the raster's tile flags.
+__device__ inline bool may_have_hole(const ViewDesc* views, const InpaintWS& ws, int t, int v) {
     if (!ws.rflags) return true;
+    const HoleTile H = tile_place(views, t, v);
+    const ViewDesc& vd = views[v];
     const int sh = vd.tile_shift;
     const int rx0 = H.tx0 >> sh, rx1 = (min(H.tx0 + kInpTile, vd.w) - 1) >> sh;
     const int ry0 = H.ty0 >> sh, ry1 = (min(H.ty0 + kInpTile, vd.h) - 1) >> sh;
@@ -167,15 +176,18 @@ __device__ inline bool may_have_hole(const ViewDesc* views, const InpaintWS& ws,
 // at a time, a thread each, from the raster's flags; neighbouring tiles go to
 // different blocks, so a large hole is spread) and then works through those
 // that may have a hole: thread (x, g) owns pixels (x, g), (x, g + 8), ...
-__global__ void __launch_bounds__(256) k_inp_tiles(const ViewDesc* __restrict__ views, InpaintWS ws, int ntiles) {
+__global__ void __launch_bounds__(256) k_inp_tiles(const ViewDesc* __restrict__ views, int nviews, InpaintWS ws) {
     __shared__ uint32_t m[kInpMaskWords];
     __shared__ u64 part[8][kInpTile];
     __shared__ uint32_t cand[8];
+    __shared__ int cand_view[256];
     const int tid = threadIdx.x, lx = tid & 31, g = tid >> 5, lane = tid & 63;
-    for (int c0 = 0; (long long)c0 * gridDim.x + blockIdx.x < ntiles; c0 += 256) {
+    for (int c0 = 0; (long long)c0 * gridDim.x + blockIdx.x < ws.ntiles; c0 += 256) {
         const long long mine = (long long)(c0 + tid) * gridDim.x + blockIdx.x;
-        const bool in = mine < ntiles;
-        const bool may = in && may_have_hole(views, ws, (int)mine);
+        const bool in = mine < ws.ntiles;
+        const int v = in ? tile_view(views, nviews, (int)mine) : 0;
+        const bool may = in && may_have_hole(views, ws, (int)mine, v);
+        cand_view[tid] = v;
         if (in && !may) ws.thole[mine] = 0;
         const u64 bal = __ballot(may);
         if ((lane & 31) == 0) cand[g] = (uint32_t)(bal >> (lane & 32));
@@ -183,9 +195,10 @@ __global__ void __launch_bounds__(256) k_inp_tiles(const ViewDesc* __restrict__ 
         for (int word = 0; word < 8; ++word) {
             uint32_t bits = cand[word];
             while (bits) {
-                const int k = c0 + word * 32 + __builtin_ctz(bits);
+                const int k = word * 32 + __builtin_ctz(bits);
                 bits &= bits - 1u;
-                const HoleTile H = tile_place(ws, k * (int)gridDim.x + (int)blockIdx.x);
+                const HoleTile H = tile_place(views, (c0 + k) * (int)gridDim.x + (int)blockIdx.x,
+                                              __builtin_amdgcn_readfirstlane(cand_view[k]));
                 const ViewDesc& vd = views[H.v];
                 bool any = false;
 #pragma unroll
@@ -209,7 +222,7 @@ __global__ void __launch_bounds__(256) k_inp_tiles(const ViewDesc* __restrict__ 
                 }
                 if (tid == 0) {
                     ws.thole[H.t] = 1;
-                    ws.htiles[atomicAdd(ws.count, 1u)] = H.t;
+                    ws.htiles[atomicAdd(ws.count, 1u)] = make_int2(H.t, H.v);
                 }
                 if (tid < kInpMaskWords) ws.mask[(size_t)H.t * kInpMaskWords + tid] = m[tid];
                 const TileMask M{m};
@@ -232,7 +245,7 @@ __global__ void __launch_bounds__(256) k_inp_tiles(const ViewDesc* __restrict__ 
                 __syncthreads();   // m, part free for the next tile
             }
         }
-        __syncthreads();   // cand free
+        __syncthreads();   // cand, cand_view free
     }
 }
 
@@ -246,8 +259,8 @@ __global__ void __launch_bounds__(256) k_inp_rows(const ViewDesc* __restrict__ v
     const int w = vd.w, h = vd.h, y0 = (int)blockIdx.x * kInpTile;
     if (y0 >= h) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nt = (w + kInpTile - 1) / kInpTile;
-    const size_t t0 = (size_t)blockIdx.y * ws.tpv + (size_t)blockIdx.x * ws.ttx;
+    const int nt = inpaint_tiles(w);
+    const size_t t0 = vd.hole_base + (size_t)blockIdx.x * nt;
     u64 carry[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) carry[k] = kNone;
@@ -307,8 +320,9 @@ __global__ void __launch_bounds__(256) k_inp_cols(const ViewDesc* __restrict__ v
     const int w = vd.w, h = vd.h, x0 = (int)blockIdx.x * kInpTile;
     if (x0 >= w) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nt = (h + kInpTile - 1) / kInpTile;
-    const size_t t0 = (size_t)blockIdx.y * ws.tpv + blockIdx.x;
+    const int nt = inpaint_tiles(h);
+    const int across = inpaint_tiles(w);
+    const size_t t0 = vd.hole_base + blockIdx.x;
     u64 carry[8], carry_own[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) { carry[k] = kNone; carry_own[k] = kNone; }
@@ -316,7 +330,7 @@ __global__ void __launch_bounds__(256) k_inp_cols(const ViewDesc* __restrict__ v
         const int e = c0 + lane;
         const bool in = e < nt;
         const int ty = FWD ? e : nt - 1 - e;
-        const size_t t = t0 + (size_t)(in ? ty : 0) * ws.ttx;
+        const size_t t = t0 + (size_t)(in ? ty : 0) * across;
         const bool hole = in && ws.thole[t] != 0;
         if (__ballot(hole) == 0ull && c0 + 64 >= nt) break;   // no later tile reads a carry
         const u64 rm = hole ? ws.rmin[t] : kNone;
@@ -367,7 +381,8 @@ __global__ void __launch_bounds__(256) k_inp_mid(const ViewDesc* __restrict__ vi
     const int tid = threadIdx.x, l = tid & 31, g = tid >> 5;
     const uint32_t n = *ws.count;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const HoleTile H = tile_place(ws, ws.htiles[i]);
+        const int2 ht = ws.htiles[i];
+        const HoleTile H = tile_place(views, ht.x, ht.y);
         const ViewDesc& vd = views[H.v];
         const int w = vd.w, h = vd.h;
         u64* const rowc = ws.rowc + (size_t)H.t * kInpTile;
@@ -446,7 +461,8 @@ __global__ void __launch_bounds__(256) k_inp_final(const ViewDesc* __restrict__ 
     const int tid = threadIdx.x, l = tid & 31, g = tid >> 5;
     const uint32_t n = *ws.count;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const HoleTile H = tile_place(ws, ws.htiles[i]);
+        const int2 ht = ws.htiles[i];
+        const HoleTile H = tile_place(views, ht.x, ht.y);
         const ViewDesc& vd = views[H.v];
         const int w = vd.w, h = vd.h;
         const u64* const rowc = ws.rowc + (size_t)H.t * kInpTile;
@@ -525,52 +541,47 @@ __global__ void k_inp_map(int w, int h, int32_t* map_out) {
 }
 
 size_t a256(size_t b) { return (b + 255) & ~(size_t)255; }
-int tiles_of(int n) { return (n + kInpTile - 1) / kInpTile; }
-size_t grid_tiles(int nviews, int max_w, int max_h) { return (size_t)nviews * tiles_of(max_w) * tiles_of(max_h); }
-
 // Sequential carving of the workspace; with a null base only its size counts.
-size_t carve(char* b, size_t npx, int nviews, int max_w, int max_h, InpaintWS& ws) {
-    const size_t nt = grid_tiles(nviews, max_w, max_h);
+size_t carve(char* b, size_t npx, size_t nt, InpaintWS& ws) {
     size_t o = 0;
     auto take = [&](size_t bytes) { char* p = b + o; o += a256(bytes); return (void*)p; };
     ws.count = (uint32_t*)take(64);
     ws.thole = (uint8_t*)take(nt);
-    ws.htiles = (int*)take(4 * nt);
+    ws.htiles = (int2*)take(8 * nt);
     ws.mask = (uint32_t*)take(4 * kInpMaskWords * nt);
     ws.rowc = (u64*)take(8 * kInpTile * nt);
     ws.colc = (u64*)take(8 * kInpTile * nt);
     ws.cola = (u64*)take(8 * kInpTile * nt);
     ws.rmin = (u64*)take(8 * nt);
     ws.px = (int2*)take(8 * npx);
-    ws.ttx = tiles_of(max_w);
-    ws.tpv = ws.ttx * tiles_of(max_h);
+    ws.ntiles = (int)nt;
     ws.rflags = nullptr;
     return o;
 }
 
 }  // namespace
 
-size_t inpaint_ws_bytes(size_t npx, int nviews, int max_w, int max_h) {
+size_t inpaint_ws_bytes(size_t npx, size_t ntiles) {
     InpaintWS ws;
-    return carve(nullptr, npx, nviews, max_w, max_h, ws);
+    return carve(nullptr, npx, ntiles, ws);
 }
 
-InpaintWS inpaint_ws_carve(void* base, size_t npx, int nviews, int max_w, int max_h) {
+InpaintWS inpaint_ws_carve(void* base, size_t npx, size_t ntiles) {
     InpaintWS ws;
-    carve((char*)base, npx, nviews, max_w, max_h, ws);   // 256-byte aligned
+    carve((char*)base, npx, ntiles, ws);   // 256-byte aligned
     return ws;
 }
 
 hipError_t launch_inpaint(const ViewDesc* views, int nviews, int max_w, int max_h, const InpaintWS& ws,
                           int32_t* map_out, hipStream_t s) {
     const dim3 b(256);
-    const size_t nt = grid_tiles(nviews, max_w, max_h);
-    const dim3 gt((unsigned)(nt < (size_t)kHoleTileBlocks ? nt : (size_t)kHoleTileBlocks));
-    const dim3 gr((unsigned)tiles_of(max_h), (unsigned)nviews), gc((unsigned)tiles_of(max_w), (unsigned)nviews);
+    const dim3 gt((unsigned)(ws.ntiles < kHoleTileBlocks ? ws.ntiles : kHoleTileBlocks));
+    const dim3 gr((unsigned)inpaint_tiles(max_h), (unsigned)nviews);
+    const dim3 gc((unsigned)inpaint_tiles(max_w), (unsigned)nviews);
     if (map_out)
         hipLaunchKernelGGL(k_inp_map, dim3((unsigned)(((size_t)max_w * max_h + 255) / 256)), b, 0, s, max_w, max_h,
                            map_out);
-    hipLaunchKernelGGL(k_inp_tiles, gt, b, 0, s, views, ws, (int)nt);
+    hipLaunchKernelGGL(k_inp_tiles, gt, b, 0, s, views, nviews, ws);
     hipLaunchKernelGGL(k_inp_rows<true>, gr, b, 0, s, views, ws);
     hipLaunchKernelGGL(k_inp_cols<true>, gc, b, 0, s, views, ws);
     hipLaunchKernelGGL(k_inp_mid, gt, b, 0, s, views, ws);

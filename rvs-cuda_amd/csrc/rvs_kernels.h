@@ -56,6 +56,7 @@ struct ViewDesc {
     int w, h, tiles_x, tiles_y;
     uint32_t tile_base;      // first global tile
     uint32_t px_base;        // first global pixel
+    uint32_t hole_base;      // first of its tiles in the inpainting's per-tile arrays
     int bitdepth;
     float blend_exp;
     float blend_inv;         // 1.0f / blend_exp
