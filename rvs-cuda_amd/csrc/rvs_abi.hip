@@ -208,11 +208,13 @@ void plan_raster(Layout& L, RasterPlan& R, int nsrc, int nviews, uint32_t ntiles
     // (tiles beyond them take the one-block-per-tile replay): a sixty-fourth
     // of the pixels, five floats per source, or what fits 16 MB, if more (where
     // sources and target are aligned every tile can be deferred: the VGA stereo
-    // pair's replay 141 -> 118 us).  Not in a fixed workspace.
+    // pair's replay 141 -> 118 us).  Not in a fixed workspace, and none at all for
+    // one source, whose tiles always take that replay.
     const uint64_t tile_px = (uint64_t)1 << (2 * shift);
     const uint64_t small = keep_max > 0 ? 16 : (16ull << 20) / (tile_px * 20 * (uint64_t)nsrc);
     uint64_t rt = (uint64_t)npx / (64 * tile_px);
     rt = rt < small ? small : rt;
+    if (nsrc == 1) rt = 0;
     // RVS_REPLAY_TILES=<n> lowers it (0: every deferred tile in order; the
     // results are the same)
     if (const char* env = std::getenv("RVS_REPLAY_TILES")) {

@@ -53,3 +53,19 @@ def test_uneven_batch_inpainted(torch_cuda, tile):
         for p in ("y", "u", "v"):
             assert np.array_equal(out[p].cpu().numpy().view(ref[p].dtype), ref[p]), (k, p)
     assert holes > 1000
+
+
+def test_one_source_keeps_no_replay_results(monkeypatch):
+    """The replay's per-source results exist for launch sets of several
+    sources only: a stage raster and a one-source view ask for none."""
+    tile = 16 * 16 * 5 * 4
+    for w, h in ((640, 480), (1366, 766)):
+        def sizes():
+            return _plan([(w, h)], 1), R.hip().rvs_raster_workspace_size(w, h, w, h, 0), _plan([(w, h)], 2)
+
+        monkeypatch.delenv("RVS_REPLAY_TILES", raising=False)
+        planned = sizes()
+        monkeypatch.setenv("RVS_REPLAY_TILES", "0")   # none at all
+        none = sizes()
+        assert none[:2] == planned[:2]
+        assert planned[2] - none[2] >= 16 * 2 * tile   # two sources: at least sixteen tiles
