@@ -34,7 +34,7 @@ typedef struct ihipStream_t* rvs_stream_t;   /* hipStream_t */
 #define RVS_E_HIP (-2)       /* HIP runtime error */
 #define RVS_E_CAPACITY (-3)  /* the binned-entry list or a workspace limit was exceeded; see rvs_last_error */
 #define RVS_E_UNSUPPORTED (-4)
-#define RVS_E_TIMEOUT (-5)   /* a bounded device-side wait gave up; the call's results are not valid */
+#define RVS_E_TIMEOUT (-5)   /* reserved: no call returns it */
 
 #define RVS_MAX_SOURCES 64
 

@@ -32,21 +32,18 @@ constexpr int kItemTv = 2 * kBinQX * kBinQY;             // floats of a kept ite
 constexpr int kItemFloats = kItemTv + 3 * kBinVerts;     // then vertices
 constexpr int kBinBlocks = 2048;    // persistent binning blocks (work items past the kept range)
 constexpr int kFlatBlocks = 65536;  // persistent blocks of the passes over the kept work items
-constexpr int kRasterGroup = 4;     // sources rasterised together in k_raster's one-phase instantiation
-constexpr int kRasterGroupMulti = 4; // sources per phase of the looping instantiation (more sources)
-// binned quads per phase whose coverage-pass results stay in LDS; with the queue below a block of the
-// looping instantiation takes 20 KB, so 7 waves per SIMD fit (1536 and 500: 6; an 8192x4096
-// panorama of eleven, three scenes, raster ms 7.7 13.7 9.0 -> 7.5 11.6 8.6)
+constexpr int kRasterGroup = 4;     // sources rasterised together: a phase of k_raster
+// binned quads per phase whose coverage-pass results stay in LDS; with the queue below a 16 x 16
+// block takes 20 KB, so that 8 waves per SIMD fit, or the 7 of the looping instantiation (1536 and
+// 500 there: 6; an 8192x4096 panorama of eleven, three scenes, raster ms 7.7 13.7 9.0 -> 7.5 11.6 8.6)
 constexpr int kRasterCache = 960;
-constexpr int kRasterCacheOne = 960; // the same for launch sets of up to kRasterGroup sources (one phase)
 // k_raster: a triangle with more pixels of a tile than this in its box is shared by the lanes of a
 // wave.  16 views of mixed sizes / an 8192x4096 equirectangular view, two scenes each, raster ms: 32
-// pixels 2.42 2.96 / 9.2 13.0; 64: 2.38 2.98 / 7.3 13.2; 96: 2.39 3.01 / 7.4 13.4; never, before the
-// other raster work: 18.1 for a view of 15.8 (magnified triangles of one size fill whole waves near
-// a pole: side by side is as good there until they exceed a wave).
+// pixels 2.42 2.96 / 9.2 13.0; 64: 2.38 2.98 / 7.3 13.2; 96: 2.39 3.01 / 7.4 13.4.  Side by side is
+// as good for triangles up to a wave's 64 pixels: magnified ones, which are of one size near a pole,
+// fill whole waves as they are.
 constexpr int kWidePx = 64;
-constexpr int kWideQueueOne = 100;  // such triangles put off per phase (in the LDS the one-phase blocks leave free)
-constexpr int kWideQueue = 100;     // the same in the looping instantiation
+constexpr int kWideQueue = 100;     // such triangles put off per phase
 constexpr int kMaxSourceSide = 65536;  // bins hold quads as (row << 16) | column; also the
                                        // largest target side (tile coordinates fit 16 bits)
 constexpr int kFallbackBlocks = 1024;

@@ -125,7 +125,11 @@ struct Quad {
     uint32_t prol;      // bit k: prol flag of slot k (transform.cpp:121-123)
 };
 
-__device__ inline bool finite3(float3 v) { return is_finite(v.x) && is_finite(v.y) && is_finite(v.z); }
+// All three finite: times 0 anything else gives a NaN (a plain sum of finite
+// numbers can overflow).
+__device__ inline bool finite3(float3 v) {
+    return __builtin_fmaf(v.z, 0.f, __builtin_fmaf(v.y, 0.f, v.x * 0.f)) == 0.f;
+}
 
 __device__ inline void quad_add(Quad& Q, int slot, float3 a, float3 b, float3 c, int out_w, int out_h, float rescale,
                                 bool validity) {
@@ -255,14 +259,10 @@ __global__ void __launch_bounds__(256) k_src_bounds(PairGeom g, int bins_x, int 
     const float inf = __builtin_inff();
     float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     // points in pairs; the minima pass over NaNs, and a point with any
-    // non-finite coordinate becomes NaNs (times 0 it gives a NaN; a plain sum
-    // of finite coordinates can overflow)
-    auto finite = [](float3 p) {
-        return __builtin_fmaf(p.z, 0.f, __builtin_fmaf(p.y, 0.f, p.x * 0.f)) == 0.f;
-    };
+    // non-finite coordinate becomes NaNs
     auto add = [&](float3 p, float3 q) {
         const float n = __builtin_nanf("");
-        const bool a = finite(p), b = finite(q);
+        const bool a = finite3(p), b = finite3(q);
         const float ps[3] = {a ? p.x : n, a ? p.y : n, a ? p.z : n}, qs[3] = {b ? q.x : n, b ? q.y : n, b ? q.z : n};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -1164,7 +1164,7 @@ struct Phase {
         return (int)a + (int)b + (int)c;
     }
 };
-static_assert(kRasterGroup == 4 && kRasterGroupMulti == 4, "a phase of four sources");
+static_assert(kRasterGroup == 4, "a phase of four sources");
 
 // The wave's share of a phase's queued triangles: each lane fetches and sets
 // up one (a single chain of loads for all of them), then the wave takes them
@@ -1358,18 +1358,17 @@ __device__ inline void encode_tile_pixel(const ViewDesc& vd, float3 c, int px, i
 }
 
 // LDS of a k_raster block.
-template <bool MULTI, int TILE>
+template <int TILE>
 struct RasterLds {
     static constexpr int NT = TILE * TILE;
     static constexpr int AREA = NT / (kTile * kTile);
-    static constexpr int GRP = MULTI ? kRasterGroupMulti : kRasterGroup;   // sources per phase
+    static constexpr int GRP = kRasterGroup;   // sources per phase
     unsigned long long key1[GRP][NT];
     uint32_t key2[GRP][NT];
     int s_deferred;       // any pixel of the tile deferred
     int s_hole;           // any pixel of the tile a hole (quality not > 0)
-    // one phase: a smaller cache keeps a 16 x 16 block within 20 KB of LDS (8 blocks per CU)
-    RasterCache<(MULTI ? kRasterCache : kRasterCacheOne) * AREA> cache;
-    typedef WideQueue<(MULTI ? kWideQueue : kWideQueueOne) * AREA> Queue;
+    RasterCache<kRasterCache * AREA> cache;
+    typedef WideQueue<kWideQueue * AREA> Queue;
     Queue wide;
     float s_tie;          // two candidates of one score met (0 / 1)
 };
@@ -1390,8 +1389,8 @@ struct RasterLds {
 // form, whose registers would otherwise spill around them.
 template <class G, int MODE, bool MULTI, int TILE, bool KEPT, bool SETTLE>
 __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
-                                            const BatchDims& d, const RasterWS& ws, RasterLds<MULTI, TILE>& L) {
-    typedef RasterLds<MULTI, TILE> Lds;
+                                            const BatchDims& d, const RasterWS& ws, RasterLds<TILE>& L) {
+    typedef RasterLds<TILE> Lds;
     typedef typename Lds::Queue Queue;
     constexpr int NT = Lds::NT, GRP = Lds::GRP;
     auto& key1 = L.key1;
@@ -1626,7 +1625,7 @@ __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const V
 template <class G, int MODE, bool MULTI, int TILE, bool SETTLE>
 __global__ void __launch_bounds__(TILE * TILE) __attribute__((amdgpu_waves_per_eu(MULTI ? (TILE > kTile ? 4 : 7) : 8)))
 k_raster(const G* __restrict__ geoms, const ViewDesc* __restrict__ views, BatchDims d, RasterWS ws) {
-    __shared__ RasterLds<MULTI, TILE> lds;
+    __shared__ RasterLds<TILE> lds;
     if (ws.status[1]) return;   // bins not filled: capacity reported to the host
     if (d.kept_geom && ws.status[4] <= d.range_cap)   // the same for the whole launch
         raster_tile<G, MODE, MULTI, TILE, true, SETTLE>(geoms, views, d, ws, lds);
@@ -2008,9 +2007,10 @@ hipError_t launch_raster(const G* geoms, const ViewDesc* views, const BatchDims&
     if (d.nsrc > kRasterGroup) {
         if (big) hipLaunchKernelGGL((k_raster<G, MODE, true, kTileBig, false>), blocks, nb, 0, s, geoms, views, d, ws);
         else hipLaunchKernelGGL((k_raster<G, MODE, true, kTile, false>), blocks, nt, 0, s, geoms, views, d, ws);
-    } else if (d.settle) {
-        if (big) hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig, true>), blocks, nb, 0, s, geoms, views, d, ws);
-        else hipLaunchKernelGGL((k_raster<G, MODE, false, kTile, true>), blocks, nt, 0, s, geoms, views, d, ws);
+    } else if (MODE == MODE_BLEND && d.settle) {
+        constexpr bool SETTLE = MODE == MODE_BLEND;   // a raw launch set never settles
+        if (big) hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig, SETTLE>), blocks, nb, 0, s, geoms, views, d, ws);
+        else hipLaunchKernelGGL((k_raster<G, MODE, false, kTile, SETTLE>), blocks, nt, 0, s, geoms, views, d, ws);
     } else {
         if (big) hipLaunchKernelGGL((k_raster<G, MODE, false, kTileBig, false>), blocks, nb, 0, s, geoms, views, d, ws);
         else hipLaunchKernelGGL((k_raster<G, MODE, false, kTile, false>), blocks, nt, 0, s, geoms, views, d, ws);
