@@ -166,11 +166,15 @@ RVS_HD uint32_t quantize_u32(float v, unsigned maxv) { return (uint32_t)cvt_i32(
 
 // Correctly rounded quotients that share a divisor: quot(n, d, recip(d)) is
 // n / d bit for bit for d in quot_den's range and |n| in quot_num's.  One
-// Newton step on a reciprocal within an ulp, then two residual corrections:
-// the same steps a correctly rounded division takes, without its scaling of
-// extreme operands (not needed in these ranges: no operand, residual or
-// result comes near the subnormals) and with the reciprocal's steps paid once
-// per divisor.  VALU issue slots on gfx950: a division 15, recip 6, quot 5.
+// Newton step on a reciprocal within an ulp, then two residual corrections
+// with fused multiply-adds (Markstein's method): the steps of a correctly
+// rounded division without its scaling of extreme operands (not needed in these
+// ranges: no operand, residual or result comes near the subnormals) and with
+// the reciprocal's steps paid once per divisor.  The Newton step rounds
+// correctly from any reciprocal within an ulp but for the divisor's largest
+// mantissa, all ones, where it has to start from the rounded one; v_rcp_f32
+// gives that (every mantissa is tested on the device).  VALU issue slots on
+// gfx950: a division 15, recip 6, quot 5.
 // Outside the ranges (a zero numerator included) quot is only near n / d.
 RVS_HD float recip(float d) {
     const float y = ff_rcp(d);
