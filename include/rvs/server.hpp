@@ -46,7 +46,9 @@ public:
     /** Closed loop: `concurrency` requests outstanding at all times. */
     int run_closed(const rvs_request* reqs, int n, int concurrency);
     const std::vector<rvs_request_stats>& stats() const { return m_stats; }
-    /** Host copy of request k's YUV planes (keep_outputs). */
+    /** Kept outputs of the last run (none without keep_outputs). */
+    size_t outputs() const { return m_out.size(); }
+    /** Host copy of request k's YUV planes, k < outputs(). */
     const std::vector<uint8_t>& output(int k) const { return m_out[k]; }
     /** Message of the last failure in the current run (empty when none). */
     std::string error() const;

@@ -185,7 +185,7 @@ int rvs_server_run_closed(void* server, const rvs_request* reqs, int n, int conc
 long long rvs_server_output(void* server, int k, void* out, size_t cap) {
     if (!server) return -1;
     rvs::Server* s = static_cast<rvs::Server*>(server);
-    if (k < 0 || k >= (int)s->stats().size()) return -1;
+    if (k < 0 || k >= (int)s->outputs()) return -1;   // none are kept without keep_outputs
     const std::vector<uint8_t>& o = s->output(k);
     if (o.empty()) return -1;
     if (out) std::memcpy(out, o.data(), o.size() < cap ? o.size() : cap);

@@ -1,4 +1,4 @@
-"""CPU: the serving binding's bytes objects -- independent of what other modules
+"""The serving binding's bytes objects -- independent of what other modules
 make of ctypes.pythonapi, which it leaves alone, and never handed out unless
 the library filled them."""
 import ctypes as C
@@ -51,7 +51,26 @@ def test_import_leaves_the_shared_functions_alone():
     subprocess.run([sys.executable, "-c", code], check=True, env=dict(os.environ, PYTHONPATH=PKG))
 
 
-@pytest.mark.parametrize("again", [b"", DATA[:100], DATA + b"x"])
+@pytest.mark.parametrize("again", [b"", DATA[:100], DATA + b"x"], ids=["gone", "shorter", "longer"])
 def test_output_that_changed_is_refused(monkeypatch, again):
     with pytest.raises(RuntimeError):
         _output(monkeypatch, _Lib(again))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("keep", [False, True])
+def test_outputs_that_are_not_kept(torch_cuda, keep):
+    print("case outputs, kept %d" % keep, flush=True)
+    import workloads as W
+    rg = W.rig("rects_640", scale=4)
+    src = W.device_sources(rg, W.render_sources(rg))
+    srv = S.Server([src], memory_budget=1 << 30, max_batch=2, slots=1, keep_outputs=keep)
+    try:
+        srv.run_closed([(0, W.device_target(rg))] * 2, 2)
+        if keep:
+            assert len(srv.output(1)) > 0
+        for k in (2, -1) if keep else (0, 1):
+            with pytest.raises(RuntimeError):
+                srv.output(k)
+    finally:
+        srv.close()
