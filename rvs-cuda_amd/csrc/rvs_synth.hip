@@ -23,8 +23,10 @@
 //      of (score bits << 32 | candidate id), and a 32-bit one, key2 = max
 //      score over the candidates that are not the maximum (the loser of each
 //      key1 update).  A pixel whose runner-up scores within 2^-18 of the
-//      winner (exact ties included), or that saw a candidate with non-finite
-//      or extreme values (key2 = all ones), is deferred.  Every other pixel
+//      winner, or that saw a candidate with non-finite or extreme values (key2
+//      = all ones), is deferred; where cameras are aligned and ties are the
+//      rule, a second pass settles those between candidates of the very same
+//      depth and validity (k_raster's SETTLE).  Every other pixel
 //      provably ends the sequential fold on the argmax (the float test errs
 //      by less than 2^-21 relative), so its winner is re-evaluated -- from
 //      the kept vertices and validity of the work item the coverage pass
@@ -427,7 +429,9 @@ __global__ void __launch_bounds__(kCullThreads) k_bin_cull(const G* __restrict__
 // and the cache lines they touch cost the wide-range scenes most of their
 // binning time.
 //
-// The counting pass is bound by VALU issue (0.55 of 0.61 T wave instructions/s).  Of its
+// The counting pass is bound by VALU issue: 0.50-0.55 T wave instructions/s of the
+// 0.72 that its mix can reach (see raster_tile), the rest being waits (its waves
+// wait 0.58 of their time, eight of them side by side).  Of its
 // 995 us for 16 mixed views before the validity's shorter form: vertices 290,
 // validities 270, boxes 200, stores of the kept state 130, tile walk 123,
 // count atomics 0 (builds that skip a part).
@@ -726,8 +730,10 @@ struct WideFill {
 // with wide ranges are shared by the block's waves, a wave each with a lane
 // per tile (an item near a pole deals thousands of tiles).  A tile that found
 // the table full while counting takes its place from the bin's cursor.
-// Bound by latency: a chain of four dependent accesses per item, so items in
-// flight matter most.  Against a block per item with a returning cursor atomic
+// Bound by latency: a chain of four dependent accesses per item and the LDS
+// atomics of lanes at one tile's cursor, so items in flight matter most (waves
+// wait 0.78 of their time, VALU and scalar units issue a quarter of their rates).
+// Against a block per item with a returning cursor atomic
 // per bin (six accesses in the chain, 8 items per CU instead of 32): 16 mixed
 // views 455 -> 280 us, an 8192x4096 panorama of eleven 1.4 -> 1.2 ms.
 template <class G>
@@ -1255,7 +1261,8 @@ struct RasterCache {
 // Candidate ids: (entry << 2) | slot, entry = index of the quad in the phase's
 // concatenated bins.  A non-deferred pixel's winner beats every other
 // candidate by more than the float test's error, so any unique id works; equal
-// scores are deferred to the in-order replay.
+// scores are deferred to the in-order replay or settled by the second pass,
+// which goes by quad and slot.
 // gt: any descriptor of the view (target-side fields: the same for all its
 // sources, so they are read once per wave).
 template <int TILE, bool KEPT, bool TIES, class G, class Cache, class Queue>
@@ -1373,8 +1380,11 @@ struct RasterLds {
     float s_tie;          // two candidates of one score met (0 / 1)
 };
 
-// One tile of k_raster.  Bound by the issue of VALU instructions (0.62 T/s of wave
-// instructions; 1024 SIMDs issue 0.61 T/s at 2.4 GHz).  Raster ms with the box and the narrowing one
+// One tile of k_raster.  Bound by the issue of VALU instructions: 0.67 T wave
+// instructions/s with 16 x 16 tiles, 0.61 with 32 x 32, of about 0.74 for its
+// mix (loops of one kind of instruction at 8 waves per SIMD reach 0.97 T/s with
+// two operands, 0.59 with three and for compares, 0.30 for reciprocals; a good
+// half of the code is of the first kind).  Raster ms with the box and the narrowing one
 // after the other, the candidates marked by exact numerators and every
 // barycentric divided out, vertex code in one body, 64-bit index arithmetic and
 // branches in the candidate and blend loops -> now: 16 views of mixed sizes
@@ -1384,9 +1394,17 @@ struct RasterLds {
 // part): resolve and blend 0.75, exact tests and keys 0.56, vertex fetch and
 // denominators 0.41, candidate scan 0.34, wide triangles 0.13, boxes 0.07, the
 // rest of a tile 0.37.  KEPT: every surviving work item keeps its vertex
-// window and validities (nearly always), so this code evaluates no vertex and
-// no validity of slots 0 and 1: a third of the instructions of the general
-// form, whose registers would otherwise spill around them.
+// window and validities, so this code evaluates no vertex and no validity of
+// slots 0 and 1: a third of the instructions of the general form, whose
+// registers would otherwise spill around them.  The general form is for launch
+// sets with items beyond the kept range: few sources and large targets never
+// have any, small targets of large sources do (1280x720 from 11 perspective
+// 2048x2048 sources keep 63 k of 110 k items).  It spills 30-45 registers, most
+// of them around the vertex evaluation; against the single body before this one
+// (2 spilled at most): that 1280x720 view 0.82 -> 0.64 ms, four of them 2.83 ->
+// 2.40, 854x480 0.65 -> 0.50, 854x480 from four panoramas 0.52 -> 0.52, and
+// 320x180 into a pole of them, one tile of 50 k quads, 1.0-1.3 -> 1.1-1.3.
+// Out-of-line vertices (9-23 spilled) are slower, 0.50 -> 0.72 ms.
 template <class G, int MODE, bool MULTI, int TILE, bool KEPT, bool SETTLE>
 __device__ __forceinline__ void raster_tile(const G* __restrict__ geoms, const ViewDesc* __restrict__ views,
                                             const BatchDims& d, const RasterWS& ws, RasterLds<TILE>& L) {
