@@ -318,7 +318,7 @@ int rvs_synthesize_noalloc(const rvs_source* srcs, int n_src, const rvs_target* 
 
 /* Per-stage device times of the last rvs_synthesize* call on the calling
  * thread, measured with HIP events recorded on its stream between the stages
- * when enabled: [0] binning (incl. culling tables built per call, culling),
+ * when enabled: [0] binning (incl. culling tables built per call, uploads, culling),
  * [1] tile raster + blend (k_raster), [2] in-order replay of deferred pixels,
  * [3] inpainting, [4] encoding; milliseconds.  After an _async call,
  * synchronise the stream first. */
